@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kSurfThreads) void k_surface(SurfArgs a, KParams<do
 
 // ---------------------------------------------------------------------------
 // Level-batched translations and pseudo-inverse applies: see gemm.hpp.
-hipError_t launch_gemm(const GemmArgs& g, hipStream_t s) { return launch_gemm_t<false>(g, s); }
+hipError_t launch_gemm(const GemmArgs& g, hipStream_t s) { return launch_gemm_seq(g, s); }
 
 // ---------------------------------------------------------------------------
 // V list.  Forward: UE samples (scaled 2^(l*deg)) scattered onto the (2np)^3

@@ -14,7 +14,6 @@
 #include <type_traits>
 
 #include "device.hpp"
-#include "gemm.hpp"
 
 namespace kifmm {
 
