@@ -25,6 +25,9 @@ constexpr int kNearChunk = 128;
 constexpr int kMaxNr = 8;
 __host__ __device__ constexpr int rhs_group(int nr) { return nr <= 1 ? 1 : nr <= 2 ? 2 : nr <= 4 ? 4 : 8; }
 constexpr int kPairStride = 224;  // 216 halo slots rounded up to a multiple of 8
+// The V-list words' padding: no target, at the halo position of a target child
+// itself (every offset slot formed from it exists).
+constexpr int kHadPadWord = 3 | 3 << 3 | 3 << 6 | (3 * 49 + 3 * 7 + 3) << 9;
 
 // Packed half spectrum of the mixed path.  The r2c layout of an n^3 real grid
 // (n = 2 np) holds (np + 1) n^2 values, frequency (ka, kb, kc), kc in [0, np].
@@ -176,10 +179,11 @@ struct VlistArgs {
   double* DC; int sz_dc;
   const int* halo; const int* hord; const uint64_t* mask; const int* tgt;
   // per group, the halo sources in V-list (node) order, padded to a multiple of 8
-  // with -1: source slot, and (halo index | offset slot of the halo index << 8)
+  // with -1: source slot, and a word (halo coordinates + 1, 3 bits each, x first;
+  // offset slot of the halo index << 9; membership of the 8 targets << 20)
   const int* psrc; const int* pslot; const int* pcnt;
   const double2* m2l;          // [343][sd*td][H]
-  double2* dspec;              // [nrhs][nsrc][sd][H]
+  double2* dspec;              // [nrhs][nsrc][sd][H], FP64: then the nonfin flags
   double2* espec;              // [nrhs][ntrg][td][H]
   // Several right-hand sides: right-hand side r of source slot s is spectrum
   // row r * nsrc + s, read from UE row r * nstride + node (likewise targets
@@ -187,6 +191,11 @@ struct VlistArgs {
   // consecutive virtual groups share their translation spectra.
   int nrhs = 1;
   int64_t nstride = 0;
+  // source spectra stored [nsrc][H][sd] instead (FP64 vector kernels, hadamard.hpp)
+  int jfast = 0;
+  // FP64: per source spectrum, whether its samples are not all finite (set by the
+  // forward transform)
+  int* nonfin = nullptr;
   // mixed Hadamard of the vector kernels (sd, td > 1): 0 one wave per group
   // reading the translation spectra per pair, 1 and 2 the halo sweep over tiles
   // of 1 or 2 groups

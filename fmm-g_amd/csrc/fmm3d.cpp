@@ -630,7 +630,7 @@ int FMM3d::build_vgroups(const std::vector<int>& order, const std::vector<int64_
     for (size_t k = 0; k < nodes.size(); k++) vg.hord[size_t(g) * 216 + k] = nodes[k].second;
   }
   vg.psrc.assign(size_t(ngrp) * kPairStride, -1);
-  vg.pslot.assign(size_t(ngrp) * kPairStride, 0);
+  vg.pslot.assign(size_t(ngrp) * kPairStride, kHadPadWord);
   vg.pcnt.assign(ngrp, 0);
 #pragma omp parallel for schedule(static)
   for (int g = 0; g < ngrp; g++) {
@@ -643,7 +643,7 @@ int FMM3d::build_vgroups(const std::vector<int>& order, const std::vector<int64_
       for (int tt = 0; tt < 8; tt++)
         if ((vg.mask[size_t(g) * 32 + tt * 4 + (r >> 6)] >> (r & 63)) & 1) tm |= 1 << tt;
       vg.psrc[size_t(g) * kPairStride + k] = vg.halo[size_t(g) * 216 + r];
-      vg.pslot[size_t(g) * kPairStride + k] = r | slot << 8 | tm << 20;
+      vg.pslot[size_t(g) * kPairStride + k] = (rx + 1) | (ry + 1) << 3 | (rz + 1) << 6 | slot << 9 | tm << 20;
     }
     vg.pcnt[g] = (k + 7) / 8 * 8;
   }
@@ -822,7 +822,7 @@ int FMM3d::upload_state() {
   {
     const size_t ns = vfwd_.src_node.size() * op.sd, nt = vfwd_.trg_node.size() * op.td;
     if (precision_ == PREC_FP64) {
-      if ((rc = check(dspec_d_.alloc(sizeof(double2) * ns * op.H), "alloc V spectra"))) return rc;
+      if ((rc = check(dspec_d_.alloc(sizeof(double2) * ns * (op.H + 1)), "alloc V spectra"))) return rc;
       if ((rc = check(espec_d_.alloc(sizeof(double2) * nt * op.H), "alloc V spectra"))) return rc;
       m2l32_d_.release(); dspec32_d_.release(); espec32_d_.release();
     } else {
@@ -1051,7 +1051,7 @@ int FMM3d::reserve_rhs(int nrhs) {
   if ((rc = grow(tval_d_, sizeof(double) * R * std::max<int64_t>(1, nt_ * TD), "alloc values"))) return rc;
   const size_t nsv = vfwd_.src_node.size() * op.sd * R, ntv = vfwd_.trg_node.size() * op.td * R;
   if (precision_ == PREC_FP64) {
-    if ((rc = grow(dspec_d_, sizeof(double2) * nsv * op.H, "alloc V spectra"))) return rc;
+    if ((rc = grow(dspec_d_, sizeof(double2) * nsv * (op.H + 1), "alloc V spectra"))) return rc;
     if ((rc = grow(espec_d_, sizeof(double2) * ntv * op.H, "alloc V spectra"))) return rc;
   } else {
     const size_t hc = size_t(spec_packed_len(op.np));

@@ -211,8 +211,8 @@ int FMM3d::build_adjoint() {
     const size_t nsrc = std::max(vfwd_.src_node.size(), vadj_.src_node.size()) * dmax;
     const size_t ntrg = std::max(vfwd_.trg_node.size(), vadj_.trg_node.size()) * dmax;
     if (precision_ == PREC_FP64) {
-      if (dspec_d_.bytes() < sizeof(double2) * nsrc * op.H &&
-          (rc = check(dspec_d_.alloc(sizeof(double2) * nsrc * op.H), "alloc V spectra")))
+      if (dspec_d_.bytes() < sizeof(double2) * nsrc * (op.H + 1) &&
+          (rc = check(dspec_d_.alloc(sizeof(double2) * nsrc * (op.H + 1)), "alloc V spectra")))
         return rc;
       if (espec_d_.bytes() < sizeof(double2) * ntrg * op.H &&
           (rc = check(espec_d_.alloc(sizeof(double2) * ntrg * op.H), "alloc V spectra")))

@@ -16,6 +16,7 @@
 
 #include "device.hpp"
 #include "gemm.hpp"
+#include "hadamard.hpp"
 
 namespace kifmm {
 
@@ -450,6 +451,7 @@ __global__ __launch_bounds__(64) void k_fft_fwd(VlistArgs v, C2* dspec) {
   for (int m = 0; m < N; m++) w[m] = v.twiddle[m];
   const int l = v.depth[node] + v.root_level;
   constexpr int R = (NSAM + 63) / 64;  // lane rounds over the surface samples
+  bool big = false;  // a sample is not finite, or so large that its spectrum may not be
   for (int s = 0; s < v.sd; s++) {
     const double scale = ldexp(1.0, int(l * v.deg[s]));
     // all rounds' samples are loaded before the grid is cleared and filled
@@ -465,6 +467,7 @@ __global__ __launch_bounds__(64) void k_fft_fwd(VlistArgs v, C2* dspec) {
       sh[r] = v.shell[qq];
       const double u = v.UE[urow * v.sz_ue + qq * v.sd + s];
       uv[r] = ok ? u * scale : 0.0;
+      if constexpr (!kPack) big = big || !(fabs(uv[r]) < 1e290);
     }
     __syncthreads();
     for (int e = lane; e < NP * NP * NP; e += 64) xb[e] = 0.0;
@@ -513,7 +516,9 @@ __global__ __launch_bounds__(64) void k_fft_fwd(VlistArgs v, C2* dspec) {
     }
     __syncthreads();
     // along z (a) -> global, frequency (ka, kb, kc); line (kb, kc)
-    C2* out = dspec + (int64_t(slot) * v.sd + s) * HS;
+    // (jfast: the DOFs of a frequency side by side)
+    C2* out = v.jfast ? dspec + int64_t(slot) * v.sd * HS + s : dspec + (int64_t(slot) * v.sd + s) * HS;
+    const int st = v.jfast ? v.sd : 1;
     auto zline = [&](int e, double2 (&o)[N]) {  // the n outputs of line e = kb h + kc
       double2 in[NP];
 #pragma unroll
@@ -540,7 +545,7 @@ __global__ __launch_bounds__(64) void k_fft_fwd(VlistArgs v, C2* dspec) {
         double2 o[N];
         zline((li / (NP - 1)) * HH + li % (NP - 1) + 1, o);
 #pragma unroll
-        for (int ka = 0; ka < N; ka++) store_c(out + li + ka * NI, o[ka]);
+        for (int ka = 0; ka < N; ka++) store_c(out + (li + ka * NI) * st, o[ka]);
       }
       for (int p = lane; p < 2 * N; p += 64) {
         const int e = (p >> 1) * HH + (p & 1) * NP;
@@ -549,73 +554,162 @@ __global__ __launch_bounds__(64) void k_fft_fwd(VlistArgs v, C2* dspec) {
         zline(e, o);
 #pragma unroll
         for (int ka = 0; ka <= NP; ka++)
-          if (!L.plane_conj(ka)) store_c(out + L.plane_index(ka), o[ka]);
+          if (!L.plane_conj(ka)) store_c(out + L.plane_index(ka) * st, o[ka]);
       }
       // the row's padding (the Hadamard sweeps it with the other frequencies)
       constexpr int NC = spec_packed_count(NP);
-      for (int q = NC + lane; q < HS; q += 64) store_c(out + q, make_double2(0, 0));
+      for (int q = NC + lane; q < HS; q += 64) store_c(out + q * st, make_double2(0, 0));
     } else {
       for (int e = lane; e < N * HH; e += 64) {
         double2 o[N];
         zline(e, o);
 #pragma unroll
-        for (int ka = 0; ka < N; ka++) store_c(out + ka * N * HH + e, o[ka]);
+        for (int ka = 0; ka < N; ka++) store_c(out + (ka * N * HH + e) * st, o[ka]);
       }
+    }
+  }
+  if constexpr (!kPack) {
+    if (v.nonfin) {
+      const int any = __any(big);
+      if (lane == 0) v.nonfin[slot] = any;
     }
   }
 }
 
-// Hadamard accumulation: one workgroup (one wave) per sibling group (the 8
-// children of a parent) and 64 frequencies; lane = frequency, each lane holds
-// the 8 targets' accumulators.  The host lists the group's sources (children
-// of the parent's colleagues) in V-list (node) order with a packed word (halo
-// index, offset slot of the halo index, 8-bit target membership), so every
-// target sees its terms in V-list order, with the 1/G factor applied per term
-// (UpwEqu2DwnChk_dgemv + cptwvv).
-template <int SD, int TD>
-__global__ __launch_bounds__(64) void k_hadamard(VlistArgs v, double nrm) {
-  const int g = blockIdx.x / v.nrhs, rh = blockIdx.x % v.nrhs;  // virtual group g * nrhs + rh
-  const int soff = rh * v.nsrc, toff = rh * v.ntrg;
-  const int f = blockIdx.y * 64 + threadIdx.x;
-  const int H = v.H;
-  const bool ok = f < H;
-  const int ff = ok ? f : 0;
-  double2 acc[8][TD];
-#pragma unroll
-  for (int t = 0; t < 8; t++)
-#pragma unroll
-    for (int i = 0; i < TD; i++) acc[t][i] = make_double2(0, 0);
-  const int cnt = v.pcnt[g];
-  const int* ps = v.psrc + int64_t(g) * kPairStride;
-  const int* pr = v.pslot + int64_t(g) * kPairStride;
-  for (int k = 0; k < cnt; k++) {
-    const int s = ps[k], word = pr[k];
-    if (s < 0) continue;
-    double2 d[SD];
-#pragma unroll
-    for (int j = 0; j < SD; j++) d[j] = v.dspec[(int64_t(s + soff) * SD + j) * H + ff];
-    const int rs = (word >> 8) & 0x3ff, tm = word >> 20;
-#pragma unroll
-    for (int tau = 0; tau < 8; tau++) {
-      if (!((tm >> tau) & 1)) continue;
-      const int slot = rs - ((tau >> 2) * 49 + ((tau >> 1) & 1) * 7 + (tau & 1));
-      const double2* T = v.m2l + int64_t(slot) * SD * TD * H;
-#pragma unroll
-      for (int i = 0; i < TD; i++)
-#pragma unroll
-        for (int j = 0; j < SD; j++) {
-          const double2 p = cmul(T[int64_t(j * TD + i) * H + ff], d[j]);
-          acc[tau][i] = make_double2(acc[tau][i].x + nrm * p.x, acc[tau][i].y + nrm * p.y);
-        }
-    }
+// Scalar-kernel Hadamard (see hadamard.hpp for the scheme).  A workgroup's table:
+// 16 frequencies (88 KB); lane = frequency x 4 target pairs, so a wave sweeps one
+// group, its source list is uniform, and a source value (read by 16 lanes as one
+// 256-byte row, the same for the 4 pairs) serves two targets a lane.  Every
+// target sees its terms in V-list order with the 1/G factor applied per term
+// (UpwEqu2DwnChk_dgemv + cptwvv); PRE: 1/G is a power of two and is taken into
+// the table.  At 4,334 groups (np 6) 2.1-2.6 ms, 3.7 with the table in L2; at 72
+// groups (np 4) 33 us, 204 before.
+constexpr int kHadF = 16;
+
+template <bool PRE>
+__global__ __launch_bounds__(1024) void k_had_scalar(VlistArgs v, double nrm, int nchunk, int nsplit) {
+  __shared__ double2 T[343 * kHadF];
+  __shared__ int lists[16][2 * kPairStride];
+  __shared__ int next;
+  if (threadIdx.x == 0) next = 0;
+  int chunk, split;
+  if (!had_block(nchunk, nsplit, chunk, split)) return;
+  const int H = v.H, f0 = chunk * kHadF;
+  const int nvg = v.ngrp * v.nrhs;
+  for (int e = threadIdx.x; e < 343 * kHadF; e += blockDim.x) {
+    double2 t = v.m2l[int64_t(e / kHadF) * H + min(f0 + e % kHadF, H - 1)];
+    if constexpr (PRE) { t.x *= nrm; t.y *= nrm; }
+    T[e] = t;
   }
-  if (!ok) return;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, fl = lane & 15, sg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const bool fok = f0 + fl < H;
+  const int f = fok ? f0 + fl : H - 1;
+  // targets 2 sg and 2 sg + 1: slot = slot of the halo index - offset of the child
+  const double2* tl = T + fl - ((sg >> 1) * 49 + (sg & 1) * 7) * kHadF;
+  const int m0 = 1 << (2 * sg);
+  int* ls = lists[wave];      // the group's source slots
+  int* lw = ls + kPairStride;  // the table positions of their halo indices, membership << 16
+  // lane l stages the list entries l, 64 + l, ... (the next group's are loaded
+  // during this one's sums); padding: the group's first source, no member
+  constexpr int NE = (kPairStride + 63) / 64;
+  int es[NE], ew[NE], cnt_n = 0, bad_n = 0;
+  auto fetch = [&](int vg) {
+    const int g = vg / v.nrhs, rh = vg % v.nrhs;
+    const int* ps = v.psrc + int64_t(g) * kPairStride;
+    const int* pw = v.pslot + int64_t(g) * kPairStride;
+    cnt_n = v.pcnt[g];
+    const int s0 = ps[0];
 #pragma unroll
-  for (int tau = 0; tau < 8; tau++) {
-    const int t = v.tgt[g * 8 + tau];
-    if (t < 0) continue;
+    for (int e = 0; e < NE; e++) {
+      const int k = lane + 64 * e < kPairStride ? lane + 64 * e : 0;
+      es[e] = ps[k];
+      ew[e] = ((pw[k] >> 9) & 0x3ff) * kHadF | (pw[k] >> 20) << 16;
+      if (es[e] < 0) es[e] = s0;
+    }
+    bad_n = 0;
 #pragma unroll
-    for (int i = 0; i < TD; i++) v.espec[(int64_t(t + toff) * TD + i) * H + f] = acc[tau][i];
+    for (int e = 0; e < NE; e++) bad_n |= v.nonfin[int64_t(rh) * v.nsrc + es[e]];
+  };
+  // an XCD's workgroups of one chunk advance through the groups side by side, so
+  // that their sources' rows are shared in its L2; a workgroup's waves take its
+  // groups from a counter (the lists' lengths differ several times over)
+  auto take = [&]() {
+    int c = 0;
+    if (lane == 0) c = atomicAdd(&next, 1);
+    c = __builtin_amdgcn_readfirstlane(c);
+    return (c / nw * nsplit + split) * nw + c % nw;
+  };
+  int vg = take();
+  if (vg < nvg) fetch(vg);
+  for (int vn; vg < nvg; vg = vn) {
+    const int g = vg / v.nrhs, rh = vg % v.nrhs;
+    const int cnt = __builtin_amdgcn_readfirstlane(cnt_n);
+    const bool bad = __any(bad_n);
+#pragma unroll
+    for (int e = 0; e < NE; e++)
+      if (lane + 64 * e < kPairStride) {
+        ls[lane + 64 * e] = es[e];
+        lw[lane + 64 * e] = ew[e];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    vn = take();
+    if (vn < nvg) fetch(vn);
+    const double2* dsp = v.dspec + int64_t(rh) * v.nsrc * H;
+    double2 acc[2] = {make_double2(0, 0), make_double2(0, 0)};
+    auto term = [&](int i, double2 t, double2 d) {
+      const double2 p = cmul(t, d);
+      if constexpr (PRE) acc[i] = cadd(acc[i], p);
+      else acc[i] = make_double2(acc[i].x + nrm * p.x, acc[i].y + nrm * p.y);
+    };
+    auto source = [&](int k) { return (dsp + int64_t(__builtin_amdgcn_readfirstlane(ls[k])) * H)[unsigned(f)]; };
+    if (!bad) {
+      // Every source's values are finite, so a source adds zeros (its spectra) to
+      // the targets that it is adjacent to and no membership is looked at.
+      // A ring of 8 sources' values (the lists are padded to 8), each reloaded for
+      // 8 sources on once it is used; the next source's spectra are read during
+      // this one's sums.
+      double2 d[8], tc[2], tn[2];
+      auto spectra = [&](int k, double2 (&t)[2]) {
+        const double2* p = tl + (lw[k] & 0xffff);
+        t[0] = p[0];
+        t[1] = p[-kHadF];
+      };
+#pragma unroll
+      for (int u = 0; u < 8; u++) d[u] = source(u);
+      spectra(0, tc);
+      for (int k = 0; k < cnt; k += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          spectra(k + u + 1, tn);
+          __builtin_amdgcn_sched_barrier(0);
+          term(0, tc[0], d[u]);
+          term(1, tc[1], d[u]);
+          __builtin_amdgcn_sched_barrier(0);
+          d[u] = source(k + 8 + u);  // (past the list: padding)
+          tc[0] = tn[0];
+          tc[1] = tn[1];
+        }
+      }
+    } else {
+      for (int k = 0; k < cnt; k++) {
+        const int w = lw[k];
+        const double2* t = tl + (w & 0xffff);
+        const double2 d = source(k);
+        if ((w >> 16) & m0) term(0, t[0], d);
+        if ((w >> 16) & (m0 << 1)) term(1, t[-kHadF], d);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the lists are read before they are replaced
+    if (!fok) continue;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int tg = v.tgt[g * 8 + 2 * sg + i];
+      if (tg >= 0) v.espec[int64_t(tg + rh * v.ntrg) * H + f] = acc[i];
+    }
   }
 }
 
@@ -832,20 +926,31 @@ static hipError_t launch_fft_inv_any(const VlistArgs& v, const C2* espec, hipStr
   return hipGetLastError();
 }
 
-hipError_t launch_vlist(const VlistArgs& v, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
-  if (v.ngrp <= 0) return hipSuccess;
-  if (v.np > kMaxNp || v.nrhs < 1) return hipErrorInvalidValue;
+hipError_t launch_vlist(const VlistArgs& v0, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+  if (v0.ngrp <= 0) return hipSuccess;
+  if (v0.np > kMaxNp || v0.nrhs < 1) return hipErrorInvalidValue;
+  VlistArgs v = v0;
+  v.jfast = 1;  // as k_had_vec reads it (one DOF: the same layout)
+  // a flag per source spectrum, behind the spectra (their buffer has one more entry a row)
+  v.nonfin = reinterpret_cast<int*>(v.dspec + int64_t(v.nsrc) * v.nrhs * v.sd * v.H);
   hipError_t e = launch_fft_fwd_any<double2>(v, v.dspec, s);
   if (e != hipSuccess) return e;
   if (e0) (void)hipEventRecord(e0, s);
   const double nrm = 1.0 / double(v.n * v.n * v.n);
-  dim3 grid(unsigned(int64_t(v.ngrp) * v.nrhs), unsigned((v.H + 63) / 64));
-  if (v.sd == 1 && v.td == 1) k_hadamard<1, 1><<<grid, dim3(64), 0, s>>>(v, nrm);
-  else if (v.sd == 4 && v.td == 3) k_hadamard<4, 3><<<grid, dim3(64), 0, s>>>(v, nrm);
-  else if (v.sd == 3 && v.td == 3) k_hadamard<3, 3><<<grid, dim3(64), 0, s>>>(v, nrm);
-  else if (v.sd == 3 && v.td == 4) k_hadamard<3, 4><<<grid, dim3(64), 0, s>>>(v, nrm);
-  else return hipErrorInvalidValue;
-  e = hipGetLastError();
+  const bool pre = (v.n & (v.n - 1)) == 0;  // 1/G is a power of two
+  if (v.sd == 1 && v.td == 1) {
+    const int nchunk = (v.H + kHadF - 1) / kHadF;
+    const HadShape h = had_shape(nchunk, int64_t(v.ngrp) * v.nrhs, 1);
+    const dim3 grid(had_grid(nchunk, h.S)), block(64 * h.W);
+    if (pre) k_had_scalar<true><<<grid, block, 0, s>>>(v, nrm, nchunk, h.S);
+    else k_had_scalar<false><<<grid, block, 0, s>>>(v, nrm, nchunk, h.S);
+    e = hipGetLastError();
+  } else {
+    if (v.sd == 4 && v.td == 3) e = launch_had_vec<4, 3>(v, pre, nrm, s);
+    else if (v.sd == 3 && v.td == 3) e = launch_had_vec<3, 3>(v, pre, nrm, s);
+    else if (v.sd == 3 && v.td == 4) e = launch_had_vec<3, 4>(v, pre, nrm, s);
+    else e = hipErrorInvalidValue;
+  }
   if (e != hipSuccess) return e;
   if (e1) (void)hipEventRecord(e1, s);
   return launch_fft_inv_any<double2>(v, v.espec, s);

@@ -727,7 +727,7 @@ __global__ __launch_bounds__(64) void k_hadamard_mx(VlistArgs v, const float2* _
     float2 d[SD];
 #pragma unroll
     for (int j = 0; j < SD; j++) d[j] = ldx((s + soff) * SD + j);
-    const int rs = (word >> 8) & 0x3ff, tm = word >> 20;
+    const int rs = (word >> 9) & 0x3ff, tm = word >> 20;
 #pragma unroll
     for (int tau = 0; tau < 8; tau++) {
       if (!((tm >> tau) & 1)) continue;

@@ -26,3 +26,18 @@ def test_level_gemm_forms(kt, coefs, np_, n, pts):
     den = W.densities(n, O.src_dof(kt), 701 + n, kind="normal")
     _, val, ref = run_pair(kt, coefs, np_, pts, pos, np.zeros_like(pos), den)
     assert rel(val, ref) <= PARITY
+
+
+# V-list sums: frequency counts that are no multiple of a chunk (np 5: 600), factors
+# 1/G that are powers of two (np 4, 8) and not, lists of very different lengths,
+# a few groups and more than a pass of a workgroup.
+@pytest.mark.parametrize("kt,coefs,np_,n,pts", [(111, [1.0, 0.25], 5, 12000, 10), (111, [1.0, 0.25], 7, 6000, 40),
+                                                (111, [1.0, 0.25], 8, 4000, 60), (321, [1.0, 0.25], 5, 2500, 20),
+                                                (511, [1.0, 0.3], 3, 6000, 8)])
+def test_vlist_forms(kt, coefs, np_, n, pts):
+    pos = W.gaussians(n, 710 + n)
+    nor = np.random.default_rng(711 + n).standard_normal((n, 3))
+    nor /= np.linalg.norm(nor, axis=1)[:, None]
+    den = W.densities(n, O.src_dof(kt), 712 + n, kind="normal")
+    _, val, ref = run_pair(kt, coefs, np_, pts, pos, nor, den, max_level=12)
+    assert rel(val, ref) <= PARITY
