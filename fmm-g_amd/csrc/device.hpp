@@ -109,9 +109,10 @@ struct NearArgs {
   const double* UE; int sz_ue;
   const double* DE; int sz_de;
   const double* tpos; double* tval;
-  // mixed Laplace near field: if set, value i (leaf order) goes to
-  // tval[tperm[i]], the caller's order (no separate scatter)
+  // if set, point i's values (leaf order) go to the place of point tperm[i], the
+  // caller's order (no separate scatter)
   const int* tperm;
+  const double* tnor = nullptr;  // transposed near field: normals of the chunks' points
   // Several right-hand sides: sden holds nrhs densities per source
   // (sden[(k * nrhs + r) * SD + s]); right-hand side r's equivalent densities
   // are rows r * nstride + node of UE and DE, and its values start at
@@ -119,8 +120,8 @@ struct NearArgs {
   // right-hand sides r0 .. r0 + nr - 1.
   int nrhs = 1, r0 = 0, nr = 1;
   int64_t nstride = 0, tstride = 0;
-  // Mixed near kernels: chunk c of the launch is chunks[order[c]] (order null:
-  // chunks[c]); with queue set, a persistent grid of workgroups takes chunk
+  // Chunk c of the launch is chunks[order[c]] (order null: chunks[c]); with queue
+  // set (mixed near kernels), a persistent grid of workgroups takes chunk
   // indices from the global counter *queue (zeroed by the launcher) instead
   // of one workgroup per chunk.
   const int* order = nullptr;
@@ -213,21 +214,13 @@ struct VlistArgs {
   int dc_store = 0;
 };
 
-// Adjoint near field (source-centric): chunk = <= kNearChunk sources of a
-// source leaf (node, tbeg = first source in leaf order, tnum); items are
-// (node << 2) | kind over the points that feed them.
-enum AdjItemKind { ADJ_TRG = 0, ADJ_DC = 1, ADJ_UC = 2 };
-struct NearTArgs {
-  const NearChunk* chunks; int nchunks;
-  const int* items;
-  const double* spos; const double* snor;            // sources, leaf order
-  const double* tpos; const double* tw;              // targets, leaf order, adjoint input (TD each)
-  const int* trg_beg; const int* trg_num;
-  const double4* geom;
-  const double* sam_dc; int n_dc; const double* DC; int sz_dc;
-  const double* sam_uc; int n_uc; const double* UC; int sz_uc;
-  double* sout;                                      // SD per source, leaf order
-};
+// Adjoint near field (source-centric): the near kernels with the roles swapped.
+// chunk = <= kNearChunk sources of a source leaf (node, tbeg = first source in
+// leaf order, tnum), tpos / tnor their positions and normals; items are (node <<
+// 2) | kind over the points that feed them: the targets of a leaf (spos, sden:
+// target positions and adjoint input) and the check surfaces of a node (sam_ue,
+// UE: DC; sam_de, DE: UC).
+enum AdjItemKind { ADJ_TRG = ITEM_EXACT, ADJ_DC = ITEM_UE, ADJ_UC = ITEM_DE };
 
 // Adjoint of M2T / L2T: the equivalent surface of `node` receives from the
 // targets of the target leaves items[ibeg..iend).
@@ -244,7 +237,7 @@ struct SurfTArgs {
 // terms, 3 values per target written to a.tval; Laplace single layer.
 hipError_t launch_near_grad(int kt, const NearArgs& a, const KParams<double>& pu, const KParams<double>& pm,
                             hipStream_t s);
-hipError_t launch_near_adjoint(int kt, const NearTArgs& a, const KParams<double>& pu, hipStream_t s);
+hipError_t launch_near_adjoint(int kt, const NearArgs& a, const KParams<double>& pu, hipStream_t s);
 hipError_t launch_surface_adjoint(int km, const SurfTArgs& a, const KParams<double>& pm, hipStream_t s);
 
 hipError_t launch_gather(const double* in, const int* perm, double* out, int64_t n, int dof, hipStream_t s);

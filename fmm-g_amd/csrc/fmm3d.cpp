@@ -255,28 +255,51 @@ NearChunk FMM3d::make_near_chunk(int B, int c, int k, int ibeg, int iend) const 
 
 const double FMM3d::kStageWeights[3] = {0.04, 0.15, 0.30};
 
+// Chunk sizes that leaves of 1 .. max_tn points are cut into: a chunk of k points
+// on copies(k) = S copies costs waves(k, S) / S sweeps of its sources plus wstage
+// for staging them; the cut minimises the sum (dynamic programming over sizes).
+// Entry n: the first chunk of the n points that are left.
+template <typename Copies, typename Waves>
+static std::vector<int> split_leaves(int max_tn, Copies copies, Waves waves, double wstage) {
+  std::vector<double> cost(size_t(max_tn) + 1, 0.0);
+  std::vector<int> pick(size_t(max_tn) + 1, 0);
+  for (int n = 1; n <= max_tn; n++) {
+    cost[n] = 1e300;
+    for (int k = 1; k <= std::min(n, kNearChunk); k++) {
+      const int S = copies(k);
+      const double c = double(waves(k, S)) / S + wstage + cost[n - k];
+      if (c < cost[n] - 1e-12) { cost[n] = c; pick[n] = k; }
+    }
+  }
+  return pick;
+}
+
+// Indices by cost, largest first, to a 4096th of the largest (equal ones in order).
+static std::vector<int> order_by_cost(const std::vector<float>& cost) {
+  constexpr int B = 4096;
+  float big = 0;
+  for (float c : cost) big = std::max(big, c);
+  const float f = big > 0 ? (B - 1) / big : 0.0f;
+  std::vector<int> beg(B + 1, 0), order(cost.size());
+  for (float c : cost) beg[size_t(B - 1 - int(c * f)) + 1]++;
+  for (int b = 0; b < B; b++) beg[size_t(b) + 1] += beg[size_t(b)];
+  for (size_t i = 0; i < cost.size(); i++) order[size_t(beg[size_t(B - 1 - int(cost[i] * f))]++)] = int(i);
+  return order;
+}
+
 // Mixed path: the near kernels put S = min(16, 128 / k) copies of a chunk's k
 // targets on the 128 lanes, so a leaf of 70 targets leaves 58 lanes idle.
 // Leaves are cut into chunks of sizes that fill the lanes: cost of a chunk =
 // (active waves) / S sweeps of its sources, plus the staging weight per wave
-// for staging them again; the cut minimises the sum (dynamic programming over
-// sizes).  The chunks are also ordered by that cost, largest first (the order
-// of the work queue).
+// for staging them again (split_leaves).  The chunks are also ordered by that
+// cost, largest first (the order of the work queue).
 void FMM3d::build_mixed_chunks() {
   const Tree& t = tree_;
-  const double wstage = kStageWeights[tune_.near_stage];
   int max_tn = 0;
   for (int B : near_leaves_) max_tn = std::max(max_tn, t.trg_num[B]);
-  std::vector<double> split_cost(size_t(max_tn) + 1, 0.0);
-  std::vector<int> split_pick(size_t(max_tn) + 1, 0);
-  for (int n = 1; n <= max_tn; n++) {
-    split_cost[n] = 1e300;
-    for (int k = 1; k <= std::min(n, kNearChunk); k++) {
-      const int S = std::min(16, kNearChunk / k);
-      const double c = double((S * k + 63) / 64) / S + 2 * wstage + split_cost[n - k];
-      if (c < split_cost[n] - 1e-12) { split_cost[n] = c; split_pick[n] = k; }
-    }
-  }
+  const std::vector<int> split_pick =
+      split_leaves(max_tn, [](int k) { return std::min(16, kNearChunk / k); },
+                   [](int k, int S) { return (S * k + 63) / 64; }, 2 * kStageWeights[tune_.near_stage]);
   const int NL = int(near_leaves_.size());
   std::vector<int64_t> moff(size_t(NL) + 1, 0);
   for (int l = 0; l < NL; l++) {
@@ -349,6 +372,13 @@ int FMM3d::build_tasks() {
   std::vector<int64_t>& ioff = near_ioff_;
   std::vector<int64_t> coff(size_t(NL) + 1, 0);
   auto x_fallback = [&](int B) { return t.trg_num[B] * TD < szDC; };  // :1249
+  // the FP64 near kernels put two points a lane on 128 / ceil(k / 2) copies, so a
+  // leaf of 70 points leaves a fifth of the lanes idle and is cut in two; staging
+  // a source again costs about 0.03 of a sweep
+  int max_tn = 0;
+  for (int B : near_leaves) max_tn = std::max(max_tn, t.trg_num[B]);
+  auto copies64 = [](int k) { return std::min(32, kNearChunk / ((k + 1) / 2)); };
+  const std::vector<int> pick = split_leaves(max_tn, copies64, [](int, int) { return 1; }, 0.03);
 #pragma omp parallel for schedule(dynamic, 256)
   for (int l = 0; l < NL; l++) {
     const int B = near_leaves[l], tn = t.trg_num[B];
@@ -356,7 +386,7 @@ int FMM3d::build_tasks() {
     if (x_fallback(B)) ni += t.off[LIST_X][B + 1] - t.off[LIST_X][B];
     if (t.depth[B] >= 2) ni++;
     ioff[size_t(l) + 1] = ni;
-    coff[size_t(l) + 1] = (tn + kNearChunk - 1) / kNearChunk;
+    for (int c = 0; c < tn; c += pick[tn - c]) coff[size_t(l) + 1]++;
   }
   for (int l = 0; l < NL; l++) {
     ioff[size_t(l) + 1] += ioff[size_t(l)];
@@ -365,6 +395,7 @@ int FMM3d::build_tasks() {
   if (ioff[size_t(NL)] > INT32_MAX) return fail(-2, "too many near-field items for 32-bit offsets");
   near_items_h_.assign(size_t(ioff[size_t(NL)]), 0);
   near_chunks_h_.assign(size_t(coff[size_t(NL)]), NearChunk{});
+  std::vector<float> near_cost(near_chunks_h_.size(), 0.0f);
   double near_exact = 0, near_all = 0;
 #pragma omp parallel for schedule(dynamic, 256) reduction(+ : near_exact, near_all)
   for (int l = 0; l < NL; l++) {
@@ -400,14 +431,18 @@ int FMM3d::build_tasks() {
       surf += op.n_sam[DE];
     }
     int64_t ci = coff[size_t(l)];
-    for (int c = 0; c < tn; c += kNearChunk)
-      near_chunks_h_[size_t(ci++)] = make_near_chunk(B, c, std::min(kNearChunk, tn - c), ibeg, ni);
+    for (int c = 0; c < tn; c += pick[tn - c]) {
+      near_cost[size_t(ci)] = float((exact + surf) / copies64(pick[tn - c]));
+      near_chunks_h_[size_t(ci++)] = make_near_chunk(B, c, pick[tn - c], ibeg, ni);
+    }
     near_exact += double(tn) * exact;
     near_all += double(tn) * (exact + surf);
   }
   work_.near_exact_pairs = near_exact;
   work_.near_pairs = near_all;
-  build_mixed_chunks();
+  near_order_h_ = order_by_cost(near_cost);
+  near_order_mx_h_.clear();
+  if (precision_ == PREC_MIXED) build_mixed_chunks();
 
   // --- S2M (:557-577) and X-list S2L (:1241-1257) ---
   s2m_tasks_h_.clear(); s2l_tasks_h_.clear(); surf_items_h_.clear(); s2m_leaf_h_.clear();
@@ -712,6 +747,7 @@ int FMM3d::upload_state() {
   KIFMM_UP(near_chunks_d_, near_chunks_h_, "upload near chunks");
   KIFMM_UP(near_chunks_mx_d_, near_chunks_mx_h_, "upload near chunks");
   KIFMM_UP(near_order_mx_d_, near_order_mx_h_, "upload near chunk order");
+  KIFMM_UP(near_order_d_, near_order_h_, "upload near chunk order");
   if (!queue_d_.bytes() && (rc = check(queue_d_.alloc(256), "alloc work-queue counter"))) return rc;
   KIFMM_UP(near_items_d_, near_items_h_, "upload near items");
   KIFMM_UP(s2m_tasks_d_, s2m_tasks_h_, "upload S2M tasks");
@@ -1124,10 +1160,6 @@ int FMM3d::prepare_rhs_steps(int nrhs) {
 int FMM3d::field(const double* d_src_den, double* d_trg_grad, hipStream_t s) {
   if (!setup_done_) return fail(-3, "field called before setup");
   if (kt_ != 111) return fail(-2, "the field pass supports the Laplace single layer (kernel 111) only");
-  if (tgrad_d_.bytes() < sizeof(double) * 3 * size_t(std::max<int64_t>(1, nt_))) {
-    int rc = check(tgrad_d_.alloc(sizeof(double) * 3 * size_t(std::max<int64_t>(1, nt_))), "alloc field");
-    if (rc) return rc;
-  }
   return evaluate_impl(d_src_den, d_trg_grad, s, true);
 }
 
@@ -1145,10 +1177,6 @@ int FMM3d::fieldFromCheckpoint(const double* d_src_den, const double* d_ue_in, d
   if (!setup_done_) return fail(-3, "field called before setup");
   if (kt_ != 111) return fail(-2, "the field pass supports the Laplace single layer (kernel 111) only");
   if (!d_ue_in) return fail(-2, "null checkpoint pointer");
-  if (tgrad_d_.bytes() < sizeof(double) * 3 * size_t(std::max<int64_t>(1, nt_))) {
-    int rc = check(tgrad_d_.alloc(sizeof(double) * 3 * size_t(std::max<int64_t>(1, nt_))), "alloc field");
-    if (rc) return rc;
-  }
   return evaluate_impl(d_src_den, d_trg_grad, s, true, 1, d_ue_in, nullptr);
 }
 
@@ -1165,7 +1193,9 @@ int FMM3d::evaluate_impl(const double* d_src_den, double* d_trg_val, hipStream_t
   int rc;
   auto mark = [&](int ph) { if (timing_) (void)hipEventRecord(events_[ph], s); };
   const bool mixed = precision_ == PREC_MIXED;
-  const bool fused_out = mixed && kt_ == 111 && !grad;
+  // the near kernels write the caller's order themselves, but for the mixed
+  // vector kernels
+  const bool fused_out = !mixed || kt_ == 111;
 
   mark(PH_INI);
   // zero the work vectors (:425-438)
@@ -1304,10 +1334,11 @@ int FMM3d::evaluate_impl(const double* d_src_den, double* d_trg_val, hipStream_t
   mark(PH_NEAR);
   NearArgs na{};
   na.chunks = near_chunks_d_.as<NearChunk>(); na.nchunks = int(near_chunks_h_.size());
+  na.order = near_order_d_.as<int>();
   if (mixed && !grad) {
     na.chunks = near_chunks_mx_d_.as<NearChunk>();
     na.nchunks = int(near_chunks_mx_h_.size());
-    if (tune_.near_mode >= 1) na.order = near_order_mx_d_.as<int>();
+    na.order = tune_.near_mode >= 1 ? near_order_mx_d_.as<int>() : nullptr;
     if (tune_.near_mode == 2) na.queue = queue_d_.as<int>();
   }
   na.items = near_items_d_.as<int>();
@@ -1322,21 +1353,17 @@ int FMM3d::evaluate_impl(const double* d_src_den, double* d_trg_val, hipStream_t
   na.nrhs = R;
   na.nstride = N;
   na.tstride = nt_ * TD;
-  if (grad) {
-    na.tval = tgrad_d_.as<double>();
-    if ((rc = check(launch_near_grad(kt_, na, pu, pm, s), "near field gradient"))) return rc;
-  } else {
-    // mixed Laplace: the near kernel writes the final values in the caller's order
-    if (fused_out) { na.tval = d_trg_val; na.tperm = tperm_d_.as<int>(); na.tstride = nt_; }
-    if ((rc = check(mixed ? launch_near_mixed(kt_, na, pu, pm, s) : launch_near(kt_, na, pu, pm, s), "near field")))
-      return rc;
-  }
+  if (fused_out) { na.tval = d_trg_val; na.tperm = tperm_d_.as<int>(); }
+  if ((rc = check(grad    ? launch_near_grad(kt_, na, pu, pm, s)
+                  : mixed ? launch_near_mixed(kt_, na, pu, pm, s)
+                          : launch_near(kt_, na, pu, pm, s),
+                  "near field")))
+    return rc;
 
   // write back (:1490-1510)
   mark(PH_FIN);
   if (!fused_out &&
-      (rc = check(launch_store_rhs(grad ? tgrad_d_.as<double>() : tval_d_.as<double>(), tperm_d_.as<int>(), d_trg_val,
-                                   nt_, grad ? 3 : TD, R, s), "scatter")))
+      (rc = check(launch_store_rhs(tval_d_.as<double>(), tperm_d_.as<int>(), d_trg_val, nt_, TD, R, s), "scatter")))
     return rc;
   mark(PH_COUNT);
   if (timing_) {
@@ -1375,7 +1402,7 @@ int FMM3d::apply_tuning(const Tuning& t) {
   if (setup_done_ && t.vec_hadamard != tune_.vec_hadamard) drop_graph();
   if (!setup_done_) { tune_ = t; trans_terms_ = t.trans; return 0; }
   const bool new_tasks = t.trans != trans_terms_;
-  const bool new_chunks = t.near_stage != tune_.near_stage;
+  const bool new_chunks = precision_ == PREC_MIXED && t.near_stage != tune_.near_stage;
   tune_ = t;
   trans_terms_ = t.trans;
   int rc = 0;

@@ -268,13 +268,14 @@ class FMM3d {
   double* splitk_for(const GemmArgs& g);
   std::vector<int> lvl_idx_h_;
   std::vector<double> scales_h_;
-  std::vector<NearChunk> near_chunks_h_;
+  std::vector<NearChunk> near_chunks_h_;     // FP64 near field and gradient
+  std::vector<int> near_order_h_;            // these by estimated cost, largest first
   std::vector<NearChunk> near_chunks_mx_h_;  // mixed near field: leaves split for full lanes
   std::vector<int> near_order_mx_h_;         // the mixed chunks by estimated cost, largest first
   std::vector<int> near_leaves_;             // evaluator leaves, node order
   std::vector<int64_t> near_ioff_;           // their item ranges in near_items_h_
   std::vector<double> sbox_;                 // per node: source bounding box (lo xyz, hi xyz)
-  DeviceBuffer near_order_mx_d_, queue_d_;
+  DeviceBuffer near_order_mx_d_, near_order_d_, queue_d_;
   std::vector<int> near_items_h_;
   std::vector<SurfTask> s2m_tasks_h_, s2l_tasks_h_;
   std::vector<int4> s2m_leaf_h_;  // S2M tasks as (leaf, first source, source count)
@@ -300,7 +301,7 @@ class FMM3d {
   DeviceBuffer lvl_idx_d_;
   DeviceBuffer sam_d_[4], shell_d_, twiddle_d_, deg_d_, ones_d_, scales_d_;
   DeviceBuffer pup_d_, pdn_d_, m2m_d_, l2l_d_, m2l_d_;
-  DeviceBuffer dspec_d_, espec_d_, tgrad_d_;
+  DeviceBuffer dspec_d_, espec_d_;
   DeviceBuffer nt_chunks_d_, nt_items_d_, ue_t_tasks_d_, de_t_tasks_d_, surf_t_items_d_, tbeg_d_, tnum_d_;
   DeviceBuffer m2mT_d_, pupT_d_, pdnT_d_, l2lT_d_;
   DeviceBuffer m2lT_d_, m2lT32_d_, deg0_d_;  // adjoint V list of the Stokes equivalent kernel

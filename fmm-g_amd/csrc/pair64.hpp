@@ -1,0 +1,119 @@
+// FP64 pair interactions of the kernels that feed no pseudo-inverse (near field,
+// its transpose, the gradient, the direct sum): 1/r from one reciprocal square
+// root instead of a square root and divisions, the kernel's constants taken into
+// the density where it is staged, and the density contracted at once (the 3 x 3
+// blocks have the form G delta_ij + H x_i x_j, so G w + H (x.w) x costs a third of
+// forming and applying the block).  Fused multiply-adds throughout: no rounding
+// order is kept here.  Closed forms: kernel3d.hpp.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "kernel3d.hpp"
+
+namespace kifmm {
+
+// 1 / sqrt(x) for normal x: the hardware estimate (about 2^-23) and one step of
+// third order, e = 1 - x y^2, y (1 + e / 2 + 3 e^2 / 8), which leaves rounding.
+__device__ __forceinline__ double rsqrt64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+__device__ __forceinline__ double dot3(double ax, double ay, double az, const double* b) {
+  return fma(ax, b[0], fma(ay, b[1], az * b[2]));
+}
+
+// Factor of density component s of kernel K (TR: of its transpose).
+template <int K>
+__device__ __forceinline__ double weight64(const KParams<double>& p, int s) {
+  if constexpr (K == 121) return -p.a;
+  else if constexpr (K == 301) return s == 3 ? p.b : p.a;
+  else if constexpr (K == 311) return p.a * p.b;
+  else if constexpr (K == 321) return -p.a;
+  else if constexpr (K == 511) return p.a * p.c;
+  else return p.a;  // 111, 312, 322; 521: the A term
+}
+// Ratio of the second constant to the one in weight64 (511: H / G, 521: C / A).
+template <int K>
+__device__ __forceinline__ double ratio64(const KParams<double>& p) {
+  if constexpr (K == 511) return p.b / p.a;
+  else if constexpr (K == 521) return p.c / p.a;
+  else return 0.0;
+}
+
+// acc += K(x; n) w for one pair, x = target - source, inv = 1/|x| (0: no
+// contribution), n the source normal, w the density with weight64 applied.
+template <int K>
+__device__ __forceinline__ void pair64(double h, double x, double y, double z, double inv, const double* n,
+                                       const double* w, double* acc) {
+  if constexpr (K == 111) {
+    acc[0] = fma(inv, w[0], acc[0]);
+  } else {
+    const double inv2 = inv * inv, inv3 = inv2 * inv;
+    if constexpr (K == 121) {
+      acc[0] = fma(inv3 * dot3(x, y, z, n), w[0], acc[0]);
+    } else if constexpr (K == 312) {
+      acc[0] = fma(inv3, dot3(x, y, z, w), acc[0]);
+    } else if constexpr (K == 322) {
+      const double nw = dot3(n[0], n[1], n[2], w), rn = dot3(x, y, z, n);
+      acc[0] = fma(inv3, fma(-3.0 * rn * inv2, dot3(x, y, z, w), nw), acc[0]);
+    } else if constexpr (K == 301 || K == 311 || K == 511) {
+      double f = dot3(x, y, z, w);
+      if constexpr (K == 301) f += w[3];
+      if constexpr (K == 511) f *= h;
+      const double g = inv3 * f;
+      acc[0] = fma(inv, w[0], fma(g, x, acc[0]));
+      acc[1] = fma(inv, w[1], fma(g, y, acc[1]));
+      acc[2] = fma(inv, w[2], fma(g, z, acc[2]));
+    } else if constexpr (K == 321) {
+      const double g = inv3 * inv2 * dot3(x, y, z, n) * dot3(x, y, z, w);
+      acc[0] = fma(g, x, acc[0]);
+      acc[1] = fma(g, y, acc[1]);
+      acc[2] = fma(g, z, acc[2]);
+    } else if constexpr (K == 521) {
+      // A (rn w + n (x.w)) + B x (n.w) + C rn (x.w) x, B = -A
+      const double rn = dot3(x, y, z, n), f = dot3(x, y, z, w), nw = dot3(n[0], n[1], n[2], w);
+      const double a = inv3 * rn, b = inv3 * f, g = fma(h * inv3 * inv2 * rn, f, -inv3 * nw);
+      acc[0] = fma(a, w[0], fma(b, n[0], fma(g, x, acc[0])));
+      acc[1] = fma(a, w[1], fma(b, n[1], fma(g, y, acc[1])));
+      acc[2] = fma(a, w[2], fma(b, n[2], fma(g, z, acc[2])));
+    }
+  }
+}
+
+// acc += K(x; n)^T w, w per target DOF, acc per source DOF.
+template <int K>
+__device__ __forceinline__ void pair64_t(double h, double x, double y, double z, double inv, const double* n,
+                                         const double* w, double* acc) {
+  if constexpr (K == 111 || K == 121 || K == 311 || K == 321 || K == 511) {
+    pair64<K>(h, x, y, z, inv, n, w, acc);  // symmetric blocks
+  } else {
+    const double inv2 = inv * inv, inv3 = inv2 * inv;
+    if constexpr (K == 312) {
+      const double g = inv3 * w[0];
+      acc[0] = fma(g, x, acc[0]);
+      acc[1] = fma(g, y, acc[1]);
+      acc[2] = fma(g, z, acc[2]);
+    } else if constexpr (K == 322) {
+      const double a = inv3 * w[0], g = -3.0 * a * inv2 * dot3(x, y, z, n);
+      acc[0] = fma(a, n[0], fma(g, x, acc[0]));
+      acc[1] = fma(a, n[1], fma(g, y, acc[1]));
+      acc[2] = fma(a, n[2], fma(g, z, acc[2]));
+    } else if constexpr (K == 521) {
+      const double rn = dot3(x, y, z, n), f = dot3(x, y, z, w), nw = dot3(n[0], n[1], n[2], w);
+      const double a = inv3 * rn, b = -inv3 * f, g = fma(h * inv3 * inv2 * rn, f, inv3 * nw);
+      acc[0] = fma(a, w[0], fma(b, n[0], fma(g, x, acc[0])));
+      acc[1] = fma(a, w[1], fma(b, n[1], fma(g, y, acc[1])));
+      acc[2] = fma(a, w[2], fma(b, n[2], fma(g, z, acc[2])));
+    } else if constexpr (K == 301) {  // 4 source DOFs
+      const double f = dot3(x, y, z, w), g = inv3 * f;
+      acc[0] = fma(inv, w[0], fma(g, x, acc[0]));
+      acc[1] = fma(inv, w[1], fma(g, y, acc[1]));
+      acc[2] = fma(inv, w[2], fma(g, z, acc[2]));
+      acc[3] = fma(h, g, acc[3]);
+    }
+  }
+}
+
+}  // namespace kifmm

@@ -41,3 +41,25 @@ def test_vlist_forms(kt, coefs, np_, n, pts):
     den = W.densities(n, O.src_dof(kt), 712 + n, kind="normal")
     _, val, ref = run_pair(kt, coefs, np_, pts, pos, nor, den, max_level=12)
     assert rel(val, ref) <= PARITY
+
+
+# Near field: chunks of one point, of odd counts, of whole 128-point rounds and just
+# above; blocks that end inside an item; more items than a staging window (thin
+# leaves beside coarse ones); separate targets; pairs under the 1e-8 cut.
+@pytest.mark.parametrize("kt", [111, 121, 311, 322, 521])
+@pytest.mark.parametrize("n,pts,gen", [(9, 4, "uniform"), (1040, 131, "uniform"), (2100, 300, "uniform"),
+                                       (6000, 3, "gauss"), (3000, 500, "close")])
+def test_near_forms(kt, n, pts, gen):
+    rng = np.random.default_rng(720 + n)
+    if gen == "gauss":
+        pos = W.gaussians(n, 721, ng=2, smin=0.002, smax=0.02)
+    else:
+        pos = W.uniform(n, 722 + n)
+    if gen == "close":
+        pos[1::7] = np.minimum(pos[::7][:len(pos[1::7])] + 3e-9, W.HI)
+    nor = rng.standard_normal((n, 3))
+    nor /= np.linalg.norm(nor, axis=1)[:, None]
+    tpos = W.uniform(n // 2 + 1, 723) if gen == "uniform" else None
+    den = rng.standard_normal(n * O.src_dof(kt))
+    _, val, ref = run_pair(kt, [1.0, 0.3], 3, pts, pos, nor, den, max_level=16, tpos=tpos)
+    assert rel(val, ref) <= PARITY
