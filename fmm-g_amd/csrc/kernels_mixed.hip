@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "device.hpp"
+#include "gemm_strip.hpp"
 
 namespace kifmm {
 
@@ -1309,7 +1310,8 @@ hipError_t launch_hadamard_mixed(const VlistArgs& v, const float2* dspec, const 
 // with the next slab prefetched into registers while the current one feeds 20
 // MFMAs per wave.  108 VGPRs and 33 KB of LDS: 4 waves per SIMD (the same tile
 // on 4 waves of ten row blocks each needed 168 VGPRs, 3 waves per SIMD, and was
-// 13% slower on the down pass).
+// 13% slower on the down pass).  Launches too small to fill the chip with tiles go to
+// k_gemm_strip.
 // With ksplit > 1, blockIdx.z = matrix * ksplit + K chunk: each chunk writes
 // its partial product to g.work, and k_splitk_reduce sums the chunks in chunk
 // order into C (deterministic), so a level with few columns still spreads over
@@ -1440,17 +1442,45 @@ __global__ void k_splitk_reduce(const double* __restrict__ work, int ks, int nco
   *dst = accumulate ? *dst + v : v;
 }
 
+// Which kernel takes a launch, all with the same bits (M x K, columns; us):
+// - split K: the strip of eight chunk waves while its workgroups x K stay within
+//   10^6, else the tile and the sum's launch (152 x 296, 64: 8 and 15; 512: 13 and
+//   20; 888 x 1,464, 64: 19 and 28; past the line 608 x 4,864, 64: 42 and 39;
+//   152 x 1,216, 2,000: 54 and 40)
+// - else strips of 16 x 8 up to two waves a SIMD (152 x 296, 512: 9, 32 x 16 strips
+//   17, tile 47; 1,280: 13, 17 and 47; past it 456 x 608, 700: 29, 28 and 88)
+// - strips of 32 x 16 up to three a SIMD (152 x 296, 6,400: 30, tile 50; 608 x 888,
+//   2,000: 91 and 130; past it 152 x 296, 12,000: 54 and 51; 608 x 888, 4,000: 151
+//   and 136)
+// - the tile.
 static hipError_t launch_gemm_mfma(const GemmArgs& g, hipStream_t s) {
   if (g.ncol <= 0) return hipSuccess;
   const bool split = g.ksplit > 1;
   if (split && (g.kchunk <= 0 || int64_t(g.ksplit) * g.kchunk < g.K || !g.work)) return hipErrorInvalidValue;
-  const int nz = (g.zoff ? g.nz : 1) * (split ? g.ksplit : 1);
-  dim3 grid(unsigned((g.M + GM_M - 1) / GM_M), unsigned((g.max_zcol + GM_N - 1) / GM_N), unsigned(nz));
-  k_gemm_mfma<<<grid, dim3(GM_T), 0, s>>>(g);
-  if (split) {
-    const int64_t n = int64_t(g.ncol) * g.M;
-    k_splitk_reduce<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(g.work, g.ksplit, g.ncol, g.M, g.cidx, g.C,
-                                                                           g.ldc, g.accumulate);
+  const int nz = g.zoff ? g.nz : 1;
+  auto strips = [&](int rows, int cols) {
+    return int64_t((g.M + rows - 1) / rows) * ((g.max_zcol + cols - 1) / cols) * nz;
+  };
+  auto strip_grid = [&](int rows, int cols) {
+    return dim3(unsigned((g.M + rows - 1) / rows), unsigned((g.max_zcol + cols - 1) / cols), unsigned(nz));
+  };
+  const bool addressable = int64_t(g.M) * g.K * 8 < (int64_t(1) << 31);  // a strip's buffer resource of A
+  constexpr int kSimds = 1024;
+  if (split && addressable && strips(16, 8) * g.K <= 1000000) {
+    k_gemm_strip<1, 2, 4, 8, true><<<strip_grid(16, 8), dim3(512), 0, s>>>(g);
+  } else if (!split && addressable && strips(16, 8) <= 2 * kSimds) {
+    k_gemm_strip<1, 2, 16, 4, false><<<strip_grid(16, 32), dim3(256), 0, s>>>(g);
+  } else if (!split && addressable && strips(32, 16) <= 3 * kSimds) {
+    k_gemm_strip<2, 4, 8, 4, false><<<strip_grid(32, 64), dim3(256), 0, s>>>(g);
+  } else {
+    dim3 grid = strip_grid(GM_M, GM_N);
+    if (split) grid.z *= unsigned(g.ksplit);
+    k_gemm_mfma<<<grid, dim3(GM_T), 0, s>>>(g);
+    if (split) {
+      const int64_t n = int64_t(g.ncol) * g.M;
+      k_splitk_reduce<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(g.work, g.ksplit, g.ncol, g.M, g.cidx, g.C,
+                                                                            g.ldc, g.accumulate);
+    }
   }
   return hipGetLastError();
 }
