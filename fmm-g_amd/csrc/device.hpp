@@ -165,6 +165,10 @@ struct GemmArgs {
   double* work;
 };
 
+// Colleagues a tile of the mixed scalar Hadamard holds (32 groups of a full level,
+// aligned, have 144; two workgroups' spectra fit a CU's LDS).
+constexpr int kM2lTileParents = 144;
+
 struct VlistArgs {
   int np, n, H, sd, td;
   int nsrc, ntrg, ngrp;
@@ -178,7 +182,7 @@ struct VlistArgs {
   const double2* twiddle;      // n entries exp(-2 pi i m/n)
   const double* UE; int sz_ue;
   double* DC; int sz_dc;
-  const int* halo; const int* hord; const uint64_t* mask; const int* tgt;
+  const int* halo; const int* tgt;
   // per group, the halo sources in V-list (node) order, padded to a multiple of 8
   // with -1: source slot, and a word (halo coordinates + 1, 3 bits each, x first;
   // offset slot of the halo index << 9; membership of the 8 targets << 20)
@@ -197,6 +201,12 @@ struct VlistArgs {
   // FP64: per source spectrum, whether its samples are not all finite (set by the
   // forward transform)
   int* nonfin = nullptr;
+  // mixed scalar Hadamard: the groups as tiles of up to 32 with their distinct
+  // colleagues (VGroups::mt_*); 0 tiles: not made.  mt_thin: fewer than 256 V-list
+  // pairs a group, of 1,512
+  int mt_tiles = 0, mt_thin = 0;
+  const int4* mt_inf = nullptr;
+  const int* mt_row = nullptr; const int* mt_idx = nullptr;
   // mixed Hadamard of the vector kernels (sd, td > 1): 0 one wave per group
   // reading the translation spectra per pair, 1 and 2 the halo sweep over tiles
   // of 1 or 2 groups

@@ -3,6 +3,7 @@
 #include "fmm3d.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -597,6 +598,7 @@ int FMM3d::build_vgroups(const std::vector<int>& order, const std::vector<int64_
   const int N = t.n_nodes;
   vg.src_node.clear(); vg.trg_node.clear(); vg.halo.clear(); vg.hord.clear(); vg.tgt.clear();
   vg.psrc.clear(); vg.pslot.clear(); vg.pcnt.clear(); vg.mask.clear();
+  vg.mt_inf.clear(); vg.mt_row.clear(); vg.mt_idx.clear();
   vg.pairs = 0;
   std::vector<int> src_slot(N, -1);
   std::map<int, int> grp;
@@ -652,6 +654,11 @@ int FMM3d::build_vgroups(const std::vector<int>& order, const std::vector<int64_
       }
     }
   if (bad) return fail(-6, "V list differs from the non-adjacent halo of its sibling group");
+  // the mixed scalar Hadamard reads the halo tables and tiles, not the lists below
+  if (precision_ == PREC_MIXED && ops_->sd == 1 && ops_->td == 1) {
+    build_m2l_tiles(vg);
+    return 0;
+  }
   // per group: halo slots ordered by node index (the V lists' order)
   vg.hord.assign(size_t(ngrp) * 216, -1);
 #pragma omp parallel for schedule(static)
@@ -683,6 +690,92 @@ int FMM3d::build_vgroups(const std::vector<int>& order, const std::vector<int64_
     vg.pcnt[g] = (k + 7) / 8 * 8;
   }
   return 0;
+}
+
+void FMM3d::build_m2l_tiles(VGroups& vg) const {
+  const int ngrp = vg.ngrp();
+  auto depth = [&](int g) {
+    for (int t = 0; t < 8; t++)
+      if (vg.tgt[size_t(g) * 8 + t] >= 0) return tree_.depth[vg.trg_node[vg.tgt[size_t(g) * 8 + t]]];
+    return -1;
+  };
+  // a colleague is a source parent and the children of it in the group's halo (those
+  // adjacent to every target of the group may be missing)
+  struct Kid { int node, mask, first; int rows[8]; };
+  std::vector<Kid> kid;            // of the tile, in order of first use
+  std::vector<int> stamp(tree_.n_nodes, -1), number(tree_.n_nodes);  // tile and number of a parent's first entry
+  uint8_t idx[27 * 32];
+  int g0 = 0, n = 0, qmask = 0, tile = 0;
+  auto find = [&](const Kid& k) -> int {
+    if (stamp[k.node] != tile) return -1;
+    if (kid[number[k.node]].mask == k.mask) return number[k.node];
+    for (size_t i = 0; i < kid.size(); i++)
+      if (kid[i].node == k.node && kid[i].mask == k.mask) return int(i);
+    return -1;
+  };
+  auto close = [&]() {
+    if (n == 0) return;
+    // numbered in the order of their rows: neighbouring groups' colleagues lie
+    // side by side in LDS
+    const int np = int(kid.size());
+    std::vector<int> ord(np), renum(np);
+    for (int k = 0; k < np; k++) ord[k] = k;
+    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return kid[x].first < kid[y].first; });
+    const size_t r0 = vg.mt_row.size(), i0 = vg.mt_idx.size();
+    vg.mt_row.resize(r0 + size_t(kM2lTileParents) * 8, -1);
+    for (int k = 0; k < np; k++) {
+      renum[ord[k]] = k;
+      for (int c = 0; c < 8; c++) vg.mt_row[r0 + size_t(c) * kM2lTileParents + k] = kid[ord[k]].rows[c];
+    }
+    vg.mt_idx.resize(i0 + 7 * 32, 0);
+    for (int q = 0; q < 27; q++)
+      for (int k = 0; k < 32; k++) {
+        const int p = idx[q * 32 + k] == 255 ? np : renum[idx[q * 32 + k]];
+        vg.mt_idx[i0 + (q / 4) * 32 + k] |= p << (8 * (q % 4));
+      }
+    vg.mt_inf.insert(vg.mt_inf.end(), {g0, n, np, qmask});
+    g0 += n;
+    n = 0; qmask = 0; tile++;
+    kid.clear();
+    std::fill(idx, idx + 27 * 32, uint8_t(255));
+  };
+  std::fill(idx, idx + 27 * 32, uint8_t(255));
+  Kid of[27];
+  for (int g = 0; g < ngrp; g++) {
+    const int* h = &vg.halo[size_t(g) * 216];
+    int fresh = 0, have = 0;
+    for (int q = 0; q < 27; q++) {
+      if (q == 13) continue;  // the parent itself: siblings are adjacent
+      Kid& k = of[q];
+      k.node = -1; k.mask = 0; k.first = INT_MAX;
+      const int* hq = h + 2 * (q / 9) * 36 + 2 * ((q / 3) % 3) * 6 + 2 * (q % 3);
+      for (int c = 0; c < 8; c++) {
+        const int r = k.rows[c] = hq[(c >> 2) * 36 + ((c >> 1) & 1) * 6 + (c & 1)];
+        if (r < 0) continue;
+        k.mask |= 1 << c;
+        k.first = std::min(k.first, r);
+      }
+      if (k.mask == 0) continue;
+      k.node = tree_.parent[vg.src_node[k.first]];
+      have |= 1 << q;
+      fresh += find(k) < 0;
+    }
+    if (n == 32 || (n > 0 && (int(kid.size()) + fresh > kM2lTileParents || depth(g) != depth(g - 1)))) close();
+    for (int q = 0; q < 27; q++) {
+      if (!((have >> q) & 1)) continue;
+      const Kid& k = of[q];
+      int i = find(k);
+      if (i < 0) {
+        i = int(kid.size());
+        kid.push_back(k);
+        if (stamp[k.node] != tile) { stamp[k.node] = tile; number[k.node] = i; }
+      }
+      idx[q * 32 + n] = uint8_t(i);
+    }
+    qmask |= have;
+    n++;
+  }
+  close();
 }
 
 int FMM3d::upload_state() {
@@ -892,12 +985,17 @@ int FMM3d::upload_vgroups(VGroups& vg) {
   KIFMM_UPV(vg.src_node_d, vg.src_node, "upload V sources");
   KIFMM_UPV(vg.trg_node_d, vg.trg_node, "upload V targets");
   KIFMM_UPV(vg.halo_d, vg.halo, "upload V halo");
-  KIFMM_UPV(vg.hord_d, vg.hord, "upload V order");
-  KIFMM_UPV(vg.psrc_d, vg.psrc, "upload V pairs");
-  KIFMM_UPV(vg.pslot_d, vg.pslot, "upload V pairs");
-  KIFMM_UPV(vg.pcnt_d, vg.pcnt, "upload V pairs");
   KIFMM_UPV(vg.tgt_d, vg.tgt, "upload V groups");
-  KIFMM_UPV(vg.mask_d, vg.mask, "upload V masks");
+  if (!vg.psrc.empty()) {
+    KIFMM_UPV(vg.psrc_d, vg.psrc, "upload V pairs");
+    KIFMM_UPV(vg.pslot_d, vg.pslot, "upload V pairs");
+    KIFMM_UPV(vg.pcnt_d, vg.pcnt, "upload V pairs");
+  }
+  if (vg.mt_tiles() > 0) {
+    KIFMM_UPV(vg.mt_inf_d, vg.mt_inf, "upload V tiles");
+    KIFMM_UPV(vg.mt_row_d, vg.mt_row, "upload V tiles");
+    KIFMM_UPV(vg.mt_idx_d, vg.mt_idx, "upload V tiles");
+  }
 #undef KIFMM_UPV
   return 0;
 }
@@ -913,10 +1011,13 @@ void FMM3d::vlist_args(VlistArgs& v, const VGroups& vg) const {
   v.src_node = vg.src_node_d.as<int>(); v.trg_node = vg.trg_node_d.as<int>();
   v.depth = depth_d_.as<int>(); v.root_level = tree_.root_level;
   v.deg = deg_d_.as<double>(); v.shell = shell_d_.as<int>(); v.twiddle = twiddle_d_.as<double2>();
-  v.halo = vg.halo_d.as<int>(); v.hord = vg.hord_d.as<int>();
+  v.halo = vg.halo_d.as<int>();
   v.psrc = vg.psrc_d.as<int>(); v.pslot = vg.pslot_d.as<int>(); v.pcnt = vg.pcnt_d.as<int>();
-  v.mask = vg.mask_d.as<uint64_t>(); v.tgt = vg.tgt_d.as<int>();
+  v.tgt = vg.tgt_d.as<int>();
   v.m2l = m2l_d_.as<double2>(); v.dspec = dspec_d_.as<double2>(); v.espec = espec_d_.as<double2>();
+  v.mt_tiles = vg.mt_tiles();
+  v.mt_thin = vg.pairs < 256.0 * vg.ngrp() ? 1 : 0;
+  v.mt_inf = vg.mt_inf_d.as<int4>(); v.mt_row = vg.mt_row_d.as<int>(); v.mt_idx = vg.mt_idx_d.as<int>();
   v.had_form = tune_.vec_hadamard;
   v.sym3 = m2l_sym3_ ? 1 : 0;
   v.mirror = m2l_mirror_ ? 1 : 0;

@@ -45,12 +45,20 @@ class DeviceBuffer {
 // V-list interactions as sibling groups: the 8 children of one parent and
 // their parent's 6^3 halo of colleague children.  Per group: halo slot ->
 // source slot (-1 empty), target child -> target slot, V membership bits, and
-// the halo slots in node order as pair lists for the ordered FP64 kernel.
+// the halo slots in node order as pair lists (all but the mixed scalar kernel).
 struct VGroups {
   std::vector<int> src_node, trg_node, halo, hord, tgt, psrc, pslot, pcnt;
   std::vector<uint64_t> mask;
   double pairs = 0;
-  DeviceBuffer src_node_d, trg_node_d, halo_d, hord_d, tgt_d, psrc_d, pslot_d, pcnt_d, mask_d;
+  // tiles of consecutive groups of one level and their distinct colleagues (source
+  // parents, by their 8 child slots): {first group, groups, colleagues, mask of
+  // the offsets with sources} of a tile, child slots [tile][8][kM2lTileParents], and the
+  // colleagues' numbers (past the last one: none), a byte an offset, four offsets a
+  // word [tile][7][32 groups]
+  std::vector<int> mt_inf, mt_row, mt_idx;
+  DeviceBuffer mt_inf_d, mt_row_d, mt_idx_d;
+  int mt_tiles() const { return int(mt_inf.size() / 4); }
+  DeviceBuffer src_node_d, trg_node_d, halo_d, tgt_d, psrc_d, pslot_d, pcnt_d;
   int ngrp() const { return int(tgt.size() / 8); }
 };
 
@@ -217,6 +225,7 @@ class FMM3d {
   int upload_state();
   int build_vgroups(const std::vector<int>& order, const std::vector<int64_t>& off, const std::vector<int>& lst,
                     bool need_evtr, VGroups& vg);
+  void build_m2l_tiles(VGroups& vg) const;
   int upload_vgroups(VGroups& vg);
   void vlist_args(VlistArgs& v, const VGroups& vg) const;
   // m2l32: FP32 translation table of the mixed path (null: the forward one)

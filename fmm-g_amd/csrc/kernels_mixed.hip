@@ -15,6 +15,7 @@
 
 #include "device.hpp"
 #include "gemm_strip.hpp"
+#include "m2l_mfma.hpp"
 
 namespace kifmm {
 
@@ -1241,6 +1242,23 @@ hipError_t launch_hadamard_mixed(const VlistArgs& v, const float2* dspec, const 
   const float nrm = float(1.0 / double(v.n * v.n * v.n));
   const int64_t nvg = int64_t(v.ngrp) * v.nrhs;  // virtual groups
   dim3 grid(unsigned(nvg), unsigned((v.H + 63) / 64));
+  // Matrix cores over tiles of groups, or the vector unit's sweep.  The former runs
+  // 512 workgroups at a time, 20 us each; one chip load of the latter takes 60 to 130
+  // us whatever is in it (up to 1,450 groups at np 6).  So launches of up to four
+  // rounds take the matrix cores, and larger ones where the tiles are filled (24
+  // groups and more of 32: uniform 300,000 points, np 6, 567 and 766 us; Gaussians
+  // 319 and 424), but thin lists (spheres; the sweep skips their empty places) only
+  // from twelve rounds on (100,000 points 231 and 268; in between 30,000 points of
+  // six spheres 119 and 103).
+  if (v.sd == 1 && v.td == 1 && v.mirror && v.mt_tiles > 0) {
+    const int64_t wgs = int64_t(v.mt_tiles) * (v.H / kMtF) * v.nrhs;
+    if (wgs <= 4 * 512 || (v.ngrp >= 24 * int64_t(v.mt_tiles) && (!v.mt_thin || wgs >= 12 * 512))) {
+      const int per_xcd = (v.mt_tiles + 7) / 8;
+      const dim3 g3(unsigned(16 * per_xcd), unsigned(v.H / (2 * kMtF)), unsigned(v.nrhs));
+      k_m2l_mfma<<<g3, dim3(64 * kMtF), 0, s>>>(v, dspec, m2l, espec, nrm, v.mt_tiles, per_xcd);
+      return hipGetLastError();
+    }
+  }
   if (v.sd == 1 && v.td == 1) {
     const int ntile = int((nvg + kTileG - 1) / kTileG);
     const int per_xcd = (ntile + 7) / 8;
