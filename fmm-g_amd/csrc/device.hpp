@@ -252,7 +252,13 @@ hipError_t launch_surface_adjoint(int km, const SurfTArgs& a, const KParams<doub
 
 hipError_t launch_gather(const double* in, const int* perm, double* out, int64_t n, int dof, hipStream_t s);
 hipError_t launch_scatter(const double* in, const int* perm, double* out, int64_t n, int dof, hipStream_t s);
-hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);
+// buffers to zero, and their lengths (0: none)
+constexpr int kZeroRanges = 5;
+struct ZeroRanges {
+  double* p[kZeroRanges] = {};
+  int64_t n[kZeroRanges] = {};
+};
+hipError_t launch_zero_ranges(const ZeroRanges& z, hipStream_t s);
 // Zero rows[k] + r * nstride (k < nrows, r < nrhs) of a row-major array of rows
 // of len doubles.
 hipError_t launch_zero_rows(double* base, const int* rows, int nrows, int len, int nrhs, int64_t nstride,

@@ -1301,25 +1301,27 @@ int FMM3d::evaluate_impl(const double* d_src_den, double* d_trg_val, hipStream_t
   mark(PH_INI);
   // zero the work vectors (:425-438)
   const int64_t NR = int64_t(N) * R;  // node rows over the right-hand sides
-  // mixed path: only the rows read before any write (the rest is stored first)
-  if (!ue_in && (rc = check(mixed ? launch_zero_rows(ue_d_.as<double>(), ue_zero_d_.as<int>(), int(ue_zero_h_.size()),
-                                                     op.dat(UE), R, N, s)
-                                  : launch_fill(ue_d_.as<double>(), NR * op.dat(UE), 0.0, s),
-                            "zero UE")))
-    return rc;
-  // mixed path: UC is read only for the contributor leaves, whose S2M task
-  // stores it whole (the fused up pass forms no UC for parents)
-  if (!mixed && (rc = check(launch_fill(uc_d_.as<double>(), NR * op.dat(UC), 0.0, s), "zero UC")))
-    return rc;
-  // DE: the downward pseudo-inverse stores it for every evaluator node at depth
-  // >= 2, and only those rows are read (L2L, L2T); the mixed path skips the fill
-  if (!mixed && (rc = check(launch_fill(de_d_.as<double>(), NR * op.dat(DE), 0.0, s), "zero DE")))
-    return rc;
-  if ((rc = check(mixed ? launch_zero_rows(dc_d_.as<double>(), dc_zero_d_.as<int>(), int(dc_zero_h_.size()), op.dat(DC),
-                                           R, N, s)
-                        : launch_fill(dc_d_.as<double>(), NR * op.dat(DC), 0.0, s),
-                  "zero DC")))
-    return rc;
+  if (mixed) {
+    // only the rows read before any write (the rest is stored first): UC is read
+    // for the contributor leaves alone, whose S2M task stores it whole (the fused up
+    // pass forms no UC for parents); DE is stored by the downward pseudo-inverse for
+    // every evaluator node at depth >= 2, and only those rows are read (L2L, L2T)
+    if (!ue_in && (rc = check(launch_zero_rows(ue_d_.as<double>(), ue_zero_d_.as<int>(), int(ue_zero_h_.size()),
+                                               op.dat(UE), R, N, s),
+                              "zero UE")))
+      return rc;
+    if ((rc = check(launch_zero_rows(dc_d_.as<double>(), dc_zero_d_.as<int>(), int(dc_zero_h_.size()), op.dat(DC), R, N,
+                                     s),
+                    "zero DC")))
+      return rc;
+  } else {
+    ZeroRanges z;
+    z.p[0] = ue_d_.as<double>(); z.n[0] = ue_in ? 0 : NR * op.dat(UE);
+    z.p[1] = uc_d_.as<double>(); z.n[1] = NR * op.dat(UC);
+    z.p[2] = de_d_.as<double>(); z.n[2] = NR * op.dat(DE);
+    z.p[3] = dc_d_.as<double>(); z.n[3] = NR * op.dat(DC);
+    if ((rc = check(launch_zero_ranges(z, s), "zero work vectors"))) return rc;
+  }
   if ((rc = check(launch_load_rhs(d_src_den, sinv_d_.as<int>(), sden_d_.as<double>(), ns_, SD, R, s),
                   "load densities")))
     return rc;

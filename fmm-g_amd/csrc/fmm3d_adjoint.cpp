@@ -266,8 +266,10 @@ int FMM3d::evaluateAdjoint(const double* d_trg_in, double* d_src_out, hipStream_
   double* bufs[4] = {ue_d_.as<double>(), uc_d_.as<double>(), de_d_.as<double>(), dc_d_.as<double>()};
   const int szs[4] = {op.dat(UE), op.dat(UC), op.dat(DE), op.dat(DC)};
 
-  for (int b = 0; b < 4; b++)
-    if ((rc = check(launch_fill(bufs[b], int64_t(N) * szs[b], 0.0, s), "zero work vectors"))) return rc;
+  ZeroRanges z;
+  for (int b = 0; b < 4; b++) { z.p[b] = bufs[b]; z.n[b] = int64_t(N) * szs[b]; }
+  z.p[4] = sden_d_.as<double>(); z.n[4] = ns_ * SD;  // the output in leaf order
+  if ((rc = check(launch_zero_ranges(z, s), "zero work vectors"))) return rc;
   if ((rc = check(launch_gather(d_trg_in, tperm_d_.as<int>(), tval_d_.as<double>(), nt_, TD, s), "gather"))) return rc;
 
   // L2T^T and M2T^T: targets -> DE / UE surfaces
@@ -353,7 +355,6 @@ int FMM3d::evaluateAdjoint(const double* d_trg_in, double* d_src_out, hipStream_
   a.tpos = spos_d_.as<double>(); a.tnor = snor_d_.as<double>();
   a.tval = sden_d_.as<double>();
   a.nstride = N;
-  if ((rc = check(launch_fill(sden_d_.as<double>(), std::max<int64_t>(1, ns_ * SD), 0.0, s), "zero output"))) return rc;
   // mixed, Laplace (a symmetric kernel): the forward FP32 near kernel
   if ((rc = check(precision_ == PREC_MIXED && kt_ == 111 ? launch_near_mixed(kt_, a, pu, pu, s)
                                                          : launch_near_adjoint(kt_, a, pu, s),
