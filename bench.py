@@ -369,15 +369,15 @@ def main():
     phases = r["phases"]
     per_phase, total_roof = phase_roofline(kt, np_, w, phases, mixed, n, n)
 
-    # roofline of the dominant kernel, the V-list Hadamard (k_m2l_tile in the
-    # mixed path, k_hadamard in FP64).  Algorithmic work: one complex
+    # roofline of the dominant kernel, the V-list Hadamard (k_m2l_mfma in the
+    # mixed path, k_had_scalar in FP64).  Algorithmic work: one complex
     # multiply-add (8 flops) per V-list (target, source) pair, frequency and
     # sd*td component.  Compulsory bytes: every source and target spectrum once
     # and the 316 translation spectra, (n_vsrc*sd + n_vtrg*td)*H*2w +
     # 316*sd*td*H*2w with w = 4 (FP32) or 8 (FP64).  The intensity (about 76
     # flop/byte in FP32) is far above the machine balance (157.3 TFLOP/s over
-    # 8 TB/s, about 20): the kernel is bound by its vector (VALU) issue, and
-    # the chip's FP32 peak is the roof.
+    # 8 TB/s, about 20): the kernel is bound by its multiply-adds (matrix
+    # cores in the mixed path, VALU in FP64), and the chip's FP32 peak is the roof.
     had_ms = phases["VListHadamard"]
     wbytes = 4 if mixed else 8
     H = spectrum_len(np_, mixed)
@@ -385,15 +385,15 @@ def main():
     alg_flops = 8.0 * w["vlist_pairs"] * H
     had_tf = alg_flops / (had_ms * 1e-3) / 1e12
     peak = PEAK_TF["fp32" if mixed else "fp64"]
-    kname = "k_m2l_tile" if mixed else "k_hadamard"
-    roofline = {"bound": "valu", "kernel": kname, "achieved": round(had_tf, 3), "peak": peak,
+    kname = "k_m2l_mfma" if mixed else "k_had_scalar"
+    roofline = {"bound": "mfma" if mixed else "valu", "kernel": kname, "achieved": round(had_tf, 3), "peak": peak,
                 "unit": "TFLOP/s", "frac": round(had_tf / peak, 4), "traffic": traffic_bytes(kname),
                 "kernel_ms": round(had_ms, 4), "algorithmic_flops": alg_flops, "algorithmic_bytes": alg_bytes,
                 "intensity_flop_per_byte": round(alg_flops / alg_bytes, 2),
                 "hbm_gbs_at_algorithmic_bytes": round(alg_bytes / (had_ms * 1e-3) / 1e9, 1)}
     near_ms = phases["EvlUList"]
     near_tf = w["near_pairs"] * 11.0 / (near_ms * 1e-3) / 1e12
-    near = {"bound": "valu", "kernel": "k_near_lap_mx" if mixed else "k_near", "achieved": round(near_tf, 3),
+    near = {"bound": "valu", "kernel": "k_near_lap_mx" if mixed else "k_near64", "achieved": round(near_tf, 3),
             "peak": peak, "unit": "TFLOP/s", "frac": round(near_tf / peak, 4), "kernel_ms": round(near_ms, 4)}
 
     cpu = None
