@@ -4,7 +4,7 @@
 //   load densities (fmm3d_eval_mpi.cpp:443-461)           k_gather
 //   S2M (:577) / X-list S2L (:1253)                       k_surface
 //   M2M, UC->UE, L2L, DC->DE (:583-592, :1371-1382)       k_gemm (level-batched, indexed columns)
-//   V-list (:1007-1059)                                   k_fft_fwd, k_hadamard, k_fft_inv
+//   V-list (:1007-1059)                                   k_fft_fwd, k_had_scalar, k_had_vec, k_fft_inv
 //   U-list S2T, W-list S2T/M2T, X-list S2T, L2T
 //     (:773-785, :1146-1165, :1249, :1383-1435)            kernels_near64.hip
 //   write back (:1490-1510)                               k_scatter

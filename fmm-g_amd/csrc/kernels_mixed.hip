@@ -1250,7 +1250,7 @@ hipError_t launch_hadamard_mixed(const VlistArgs& v, const float2* dspec, const 
   // 319 and 424), but thin lists (spheres; the sweep skips their empty places) only
   // from twelve rounds on (100,000 points 231 and 268; in between 30,000 points of
   // six spheres 119 and 103).
-  if (v.sd == 1 && v.td == 1 && v.mirror && v.mt_tiles > 0) {
+  if (v.sd == 1 && v.td == 1 && v.mirror && v.mt_tiles > 0 && v.nrhs <= 65535) {
     const int64_t wgs = int64_t(v.mt_tiles) * (v.H / kMtF) * v.nrhs;
     if (wgs <= 4 * 512 || (v.ngrp >= 24 * int64_t(v.mt_tiles) && (!v.mt_thin || wgs >= 12 * 512))) {
       const int per_xcd = (v.mt_tiles + 7) / 8;
