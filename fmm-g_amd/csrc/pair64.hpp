@@ -24,21 +24,24 @@ __device__ __forceinline__ double dot3(double ax, double ay, double az, const do
   return fma(ax, b[0], fma(ay, b[1], az * b[2]));
 }
 
-// Factor of density component s of kernel K (TR: of its transpose).
+// Factor of density component s of kernel K and of its transpose.  The Navier
+// kernels' is the constant that no nu makes zero (511: H / mu, 521: C); the other
+// one, zero at nu = 3/4 (G) and nu = 1/2 (A), stands as its ratio to it.
 template <int K>
 __device__ __forceinline__ double weight64(const KParams<double>& p, int s) {
   if constexpr (K == 121) return -p.a;
   else if constexpr (K == 301) return s == 3 ? p.b : p.a;
   else if constexpr (K == 311) return p.a * p.b;
   else if constexpr (K == 321) return -p.a;
-  else if constexpr (K == 511) return p.a * p.c;
-  else return p.a;  // 111, 312, 322; 521: the A term
+  else if constexpr (K == 511) return p.b * p.c;
+  else if constexpr (K == 521) return p.c;
+  else return p.a;  // 111, 312, 322
 }
-// Ratio of the second constant to the one in weight64 (511: H / G, 521: C / A).
+// Ratio of the other constant to the one in weight64 (511: G / H, 521: A / C).
 template <int K>
 __device__ __forceinline__ double ratio64(const KParams<double>& p) {
-  if constexpr (K == 511) return p.b / p.a;
-  else if constexpr (K == 521) return p.c / p.a;
+  if constexpr (K == 511) return p.a / p.b;
+  else if constexpr (K == 521) return p.a / p.c;
   else return 0.0;
 }
 
@@ -61,11 +64,10 @@ __device__ __forceinline__ void pair64(double h, double x, double y, double z, d
     } else if constexpr (K == 301 || K == 311 || K == 511) {
       double f = dot3(x, y, z, w);
       if constexpr (K == 301) f += w[3];
-      if constexpr (K == 511) f *= h;
-      const double g = inv3 * f;
-      acc[0] = fma(inv, w[0], fma(g, x, acc[0]));
-      acc[1] = fma(inv, w[1], fma(g, y, acc[1]));
-      acc[2] = fma(inv, w[2], fma(g, z, acc[2]));
+      const double g = inv3 * f, c = K == 511 ? h * inv : inv;
+      acc[0] = fma(c, w[0], fma(g, x, acc[0]));
+      acc[1] = fma(c, w[1], fma(g, y, acc[1]));
+      acc[2] = fma(c, w[2], fma(g, z, acc[2]));
     } else if constexpr (K == 321) {
       const double g = inv3 * inv2 * dot3(x, y, z, n) * dot3(x, y, z, w);
       acc[0] = fma(g, x, acc[0]);
@@ -74,7 +76,7 @@ __device__ __forceinline__ void pair64(double h, double x, double y, double z, d
     } else if constexpr (K == 521) {
       // A (rn w + n (x.w)) + B x (n.w) + C rn (x.w) x, B = -A
       const double rn = dot3(x, y, z, n), f = dot3(x, y, z, w), nw = dot3(n[0], n[1], n[2], w);
-      const double a = inv3 * rn, b = inv3 * f, g = fma(h * inv3 * inv2 * rn, f, -inv3 * nw);
+      const double hi = h * inv3, a = hi * rn, b = hi * f, g = fma(inv3 * inv2 * rn, f, -hi * nw);
       acc[0] = fma(a, w[0], fma(b, n[0], fma(g, x, acc[0])));
       acc[1] = fma(a, w[1], fma(b, n[1], fma(g, y, acc[1])));
       acc[2] = fma(a, w[2], fma(b, n[2], fma(g, z, acc[2])));
@@ -102,7 +104,7 @@ __device__ __forceinline__ void pair64_t(double h, double x, double y, double z,
       acc[2] = fma(a, n[2], fma(g, z, acc[2]));
     } else if constexpr (K == 521) {
       const double rn = dot3(x, y, z, n), f = dot3(x, y, z, w), nw = dot3(n[0], n[1], n[2], w);
-      const double a = inv3 * rn, b = -inv3 * f, g = fma(h * inv3 * inv2 * rn, f, inv3 * nw);
+      const double hi = h * inv3, a = hi * rn, b = -hi * f, g = fma(inv3 * inv2 * rn, f, hi * nw);
       acc[0] = fma(a, w[0], fma(b, n[0], fma(g, x, acc[0])));
       acc[1] = fma(a, w[1], fma(b, n[1], fma(g, y, acc[1])));
       acc[2] = fma(a, w[2], fma(b, n[2], fma(g, z, acc[2])));
