@@ -225,8 +225,12 @@ int FMM3d::setup_prepare(bool device_tree) {
 }
 
 // A near-field chunk of leaf B: targets [c, c + k) of the leaf, items
-// [ibeg, iend); own / unchk from the bounding boxes (see NearChunk).
-NearChunk FMM3d::make_near_chunk(int B, int c, int k, int ibeg, int iend) const {
+// [ibeg, iend); own / unchk from the bounding boxes (see NearChunk).  The targets
+// lie a box side or more away from the surfaces in their items (the DE surface of
+// their own box, UE surfaces of nodes that do not touch it); surf: boxes so small
+// that this could fall under the pair cut, or vanish in the coordinates' rounding,
+// keep the cut too (FP64 kernels).
+NearChunk FMM3d::make_near_chunk(int B, int c, int k, int ibeg, int iend, bool surf) const {
   const Tree& t = tree_;
   NearChunk ch{B, t.trg_beg[B] + c, k, ibeg, iend};
   double tb[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
@@ -237,10 +241,16 @@ NearChunk FMM3d::make_near_chunk(int B, int c, int k, int ibeg, int iend) const 
       tb[3 + d] = std::max(tb[3 + d], tpos_[3 * o + d]);
     }
   }
+  double far = t.rad0;  // largest coordinate of the domain
+  for (int d = 0; d < 3; d++) far = std::max(far, std::abs(t.ctr[d]) + t.rad0);
+  const double rmin = surf ? std::max(1e-7, 1e-13 * far) : 0.0;
   bool sep = true;
   for (int i = ibeg; i < iend && sep; i++) {
     const int code = near_items_h_[size_t(i)], A = code >> 2;
-    if ((code & 3) != ITEM_EXACT) continue;  // surfaces of non-adjacent nodes or the DE surface
+    if ((code & 3) != ITEM_EXACT) {
+      if (t.radius(A) < rmin) sep = false;
+      continue;
+    }
     if (A == B && ch.own < 0) { ch.own = i - ibeg; continue; }
     const double* bx = &sbox_[size_t(A) * 6];
     double d2 = 0;
@@ -325,7 +335,7 @@ void FMM3d::build_mixed_chunks() {
       const int k = split_pick[tn - c];
       const int S = std::min(16, kNearChunk / k);
       cost[size_t(mi)] = double((S * k + 63) / 64) / S * src;
-      near_chunks_mx_h_[size_t(mi++)] = make_near_chunk(B, c, k, ibeg, iend);
+      near_chunks_mx_h_[size_t(mi++)] = make_near_chunk(B, c, k, ibeg, iend, false);
       c += k;
     }
   }
@@ -434,7 +444,7 @@ int FMM3d::build_tasks() {
     int64_t ci = coff[size_t(l)];
     for (int c = 0; c < tn; c += pick[tn - c]) {
       near_cost[size_t(ci)] = float((exact + surf) / copies64(pick[tn - c]));
-      near_chunks_h_[size_t(ci++)] = make_near_chunk(B, c, pick[tn - c], ibeg, ni);
+      near_chunks_h_[size_t(ci++)] = make_near_chunk(B, c, pick[tn - c], ibeg, ni, true);
     }
     near_exact += double(tn) * exact;
     near_all += double(tn) * (exact + surf);

@@ -220,7 +220,7 @@ class FMM3d {
   void drop_graph();
   int build_tasks();
   int retask();  // task tables and device state again (after a change of translations)
-  NearChunk make_near_chunk(int B, int c, int k, int ibeg, int iend) const;
+  NearChunk make_near_chunk(int B, int c, int k, int ibeg, int iend, bool surf) const;
   void build_mixed_chunks();
   int upload_state();
   int build_vgroups(const std::vector<int>& order, const std::vector<int64_t>& off, const std::vector<int>& lst,

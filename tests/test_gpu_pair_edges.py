@@ -1,0 +1,45 @@
+"""GPU: the FP64 pair sums at the edges of their range, against the CPU oracle (relative
+2-norm 1e-12, the FP64 parity bar) and by the transposed pass.
+"""
+import numpy as np
+import pytest
+
+import kifmm
+import oracle as O
+from kifmm import workloads as W
+from test_gpu_adjoint import dual_gap
+from test_gpu_parity import PARITY, rel, run_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def deep_boxes(n, seed):
+    """n points, the first eleven in two boxes of level 27 (7.5e-9 wide): three in a
+    leaf, eight in a split one beside it, in the child box that does not touch the
+    leaf.  Of that child the leaf sees the equivalent surface, of its own box the
+    outer one, both closer than the 1e-8 pair cut in part; its only source list
+    entry is itself."""
+    pos = W.uniform(n, seed)
+    p = np.floor(pos[0] * 2.0 ** 26)
+    rng = np.random.default_rng(seed + 1)
+    pos[:3] = (2 * p + rng.random((3, 3))) * 2.0 ** -27
+    for k in range(8):
+        child = 2 * (4 * p + (3, 1, 0)) + (k >> 2, (k >> 1) & 1, k & 1)
+        pos[3 + k] = (child + rng.random(3)) * 2.0 ** -29
+    return pos
+
+
+@pytest.mark.parametrize("kt", [111, 121, 311])
+def test_surfaces_under_the_pair_cut(kt):
+    n = 400
+    rng = np.random.default_rng(770)
+    pos = deep_boxes(n, 771)
+    nor = rng.standard_normal((n, 3))
+    nor /= np.linalg.norm(nor, axis=1)[:, None]
+    den = rng.standard_normal(n * O.src_dof(kt))
+    f, val, ref = run_pair(kt, [1.0, 0.25], 4, 6, pos, nor, den)
+    assert f.tree()["max_depth"] == 29
+    deep = 3 * O.trg_dof(kt)
+    assert np.abs(val[:deep] - ref[:deep]).max() <= 1e-12 * np.abs(ref).max()
+    assert rel(val, ref) <= PARITY
+    assert dual_gap(f, 772) < 1e-12
