@@ -299,9 +299,10 @@ struct DirectPlan {
 };
 // nchunk == 0 when the workspace capacity cannot hold one chunk's partial sums.
 DirectPlan plan_direct(int64_t ns, int nt, int td, int64_t cap_doubles);
+// src_r2: the largest |source|^2 there can be.
 hipError_t launch_direct(int kt, const KParams<double>& p, int64_t ns, const double* spos, const double* snor,
-                         const int* sperm, const double* sden, int nt, const double* tpos, const DirectPlan& d,
-                         double* work, double* tval, hipStream_t s);
+                         const int* sperm, const double* sden, int nt, const double* tpos, double src_r2,
+                         const DirectPlan& d, double* work, double* tval, hipStream_t s);
 
 // Library-held scratch of kScratchDoubles doubles per GPU (a static device
 // array, no allocation): its device address on the current GPU, looked up on

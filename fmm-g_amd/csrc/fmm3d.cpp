@@ -1635,8 +1635,10 @@ int FMM3d::directNoAlloc(const double* d_src_den, int nchk, const double* d_chk_
 int FMM3d::direct_with(const double* d_src_den, int nchk, const double* d_chk_pos, double* d_chk_val,
                        const DirectPlan& d, double* work, hipStream_t s) {
   const KParams<double> pu = make_params(kt_, coefs_.data());
+  double src_r2 = 0;
+  for (int k = 0; k < 3; k++) src_r2 += std::pow(std::abs(tree_.ctr[k]) + tree_.rad0, 2);
   return check(launch_direct(kt_, pu, ns_, spos_d_.as<double>(), snor_d_.as<double>(), sperm_d_.as<int>(), d_src_den,
-                             nchk, d_chk_pos, d, work, d_chk_val, s),
+                             nchk, d_chk_pos, src_r2, d, work, d_chk_val, s),
                "direct sum");
 }
 

@@ -846,12 +846,14 @@ hipError_t launch_fft_inv32(const VlistArgs& v, const float2* espec, hipStream_t
 // Each chunk writes its partial sums to part[y][target][TD]; k_direct_sum adds
 // the chunks in chunk order (deterministic for a given chunk count).  4,096
 // targets, 1M sources, Laplace: 2.3 ms (5.7 with one target a thread, square root
-// and division).
+// and division).  The reciprocal square root has no value where r^2 overflows: a
+// target (or a domain, src_r2 its largest squared coordinate) that far away is summed
+// again with the kernel block, which gives 0 there.
 template <int KT, int Q>
 __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t ns, int64_t chunk,
                                                      const double* __restrict__ spos, const double* __restrict__ snor,
                                                      const int* __restrict__ sperm, const double* __restrict__ sden,
-                                                     int nt, const double* __restrict__ tpos,
+                                                     int nt, const double* __restrict__ tpos, double src_r2,
                                                      double* __restrict__ part) {
   constexpr int SD = src_dof(KT), TD = trg_dof(KT);
   constexpr bool NOR = needs_normals_ct(KT);
@@ -901,9 +903,25 @@ __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t 
 #pragma unroll
   for (int q = 0; q < Q; q++) {
     const int i = (int(blockIdx.x) * Q + q) * 256 + tid;
-    if (i < nt)
+    if (i >= nt) continue;
+    if (!(tx[q] * tx[q] + ty[q] * ty[q] + tz[q] * tz[q] + src_r2 < 1e300)) {
 #pragma unroll
-      for (int d = 0; d < TD; d++) part[(int64_t(blockIdx.y) * nt + i) * TD + d] = acc[q][d];
+      for (int d = 0; d < TD; d++) acc[q][d] = 0.0;
+#pragma unroll 1
+      for (int64_t j = j0; j < j1; j++) {
+        double blk[SD * TD], n[3] = {0.0, 0.0, 0.0};
+        if constexpr (NOR)
+          for (int d = 0; d < 3; d++) n[d] = snor[3 * j + d];
+        kblock<KT, double>(p, tx[q] - spos[3 * j], ty[q] - spos[3 * j + 1], tz[q] - spos[3 * j + 2], n[0], n[1], n[2], blk);
+        const double* w = sden + int64_t(sperm[j]) * SD;
+#pragma unroll
+        for (int d = 0; d < TD; d++)
+#pragma unroll
+          for (int e = 0; e < SD; e++) acc[q][d] += blk[d * SD + e] * w[e];
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < TD; d++) part[(int64_t(blockIdx.y) * nt + i) * TD + d] = acc[q][d];
   }
 }
 
@@ -963,15 +981,15 @@ DirectPlan plan_direct(int64_t ns, int nt, int td, int64_t cap_doubles) {
 }
 
 hipError_t launch_direct(int kt, const KParams<double>& p, int64_t ns, const double* spos, const double* snor,
-                         const int* sperm, const double* sden, int nt, const double* tpos, const DirectPlan& d,
-                         double* work, double* tval, hipStream_t s) {
+                         const int* sperm, const double* sden, int nt, const double* tpos, double src_r2,
+                         const DirectPlan& d, double* work, double* tval, hipStream_t s) {
   if (nt <= 0) return hipSuccess;
   if (d.nchunk <= 0 || !work || d.chunk <= 0 || int64_t(d.nchunk) * d.chunk < ns) return hipErrorInvalidValue;
   const int q = direct_targets(nt);
   const dim3 grid(unsigned((nt + 256 * q - 1) / (256 * q)), unsigned(d.nchunk));
   switch (kt) {
 #define KIFMM_CASE_Q(K, Q) \
-    k_direct_part<K, Q><<<grid, dim3(256), 0, s>>>(p, ns, d.chunk, spos, snor, sperm, sden, nt, tpos, work)
+    k_direct_part<K, Q><<<grid, dim3(256), 0, s>>>(p, ns, d.chunk, spos, snor, sperm, sden, nt, tpos, src_r2, work)
 #define KIFMM_CASE(K)                   \
     case K:                             \
       if (q == 4) KIFMM_CASE_Q(K, 4);   \

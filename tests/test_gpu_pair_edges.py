@@ -43,3 +43,26 @@ def test_surfaces_under_the_pair_cut(kt):
     assert np.abs(val[:deep] - ref[:deep]).max() <= 1e-12 * np.abs(ref).max()
     assert rel(val, ref) <= PARITY
     assert dual_gap(f, 772) < 1e-12
+
+
+@pytest.mark.parametrize("kt", [111, 121, 311, 312, 321, 521])
+def test_direct_far_targets(gpu, kt):
+    """Check targets so far that r^2 (and earlier its powers) overflow."""
+    import torch
+    n = 700
+    pos, nor = W.spheres(n, 774, nsph=3)
+    den = np.random.default_rng(775).standard_normal(n * O.src_dof(kt))
+    f = kifmm.FMM3d(kt, [1.0, 0.3], 4, 64, 30)
+    f.set_points(pos, nor)
+    f.setup()
+    chk = np.random.default_rng(776).standard_normal((1030, 3))
+    for k, s in enumerate((1e60, 1e100, 1e153, 1.3e154, 1e155, 1e200, 1e300)):
+        chk[k::9] *= s
+    out = torch.empty(len(chk) * f.trg_dof, dtype=torch.float64, device="cuda:0")
+    f.direct_device(torch.from_numpy(den).cuda(), torch.from_numpy(chk).cuda(), out)
+    ref = O.direct(kt, [1.0, 0.3], pos, nor, den, chk)
+    assert np.isfinite(ref).all()
+    out = out.cpu().numpy()
+    assert rel(out, ref) <= PARITY
+    far = np.abs(np.repeat(chk, f.trg_dof, axis=0)).max(1) > 1e150
+    assert np.abs(out[far] - ref[far]).max() <= 1e-140
