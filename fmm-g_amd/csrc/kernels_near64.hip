@@ -31,6 +31,10 @@ namespace kifmm {
 enum Near64Mode { NEAR64_VAL = 0, NEAR64_GRAD = 1, NEAR64_T = 2 };
 constexpr int kN64Threads = 128, kN64Win = 128, kN64Copies = 32;
 typedef const __attribute__((address_space(1))) double* n64_ptr;
+// Offset of an item's source `row` among rows of `len` values.  64 bits: one leaf's
+// densities over all right-hand sides may pass 2^32 values.
+__host__ __device__ constexpr int64_t n64_off(unsigned row, unsigned len) { return int64_t(uint64_t(row) * len); }
+static_assert(n64_off(131071, 3 * 10950) == 4305682350 && n64_off(1500000000, 3) == 4500000000, "past 32 bits");
 
 template <int KT, int NR, int MODE>
 struct Near64 {
@@ -167,19 +171,19 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
             const int kind = sh.kind[lo[e]];
             const bool ex = kind == ITEM_EXACT;
             const auto& it = sh.item[lo[e]];
-            const n64_ptr ps = it.pos + ((off << 1) + off);
+            const n64_ptr ps = it.pos + n64_off(off, 3);
             const double w = it.cw[3];
             rec[0] = fma(w, ps[0], it.cw[0]);
             rec[1] = fma(w, ps[1], it.cw[1]);
             rec[2] = fma(w, ps[2], it.cw[2]);
             if constexpr (C::SNOR) {
               if (pass == 0) {
-                const n64_ptr pn_ = it.nor + ((off << 1) + off);
+                const n64_ptr pn_ = it.nor + n64_off(off, 3);
                 rec[3] = pn_[0]; rec[4] = pn_[1]; rec[5] = pn_[2];
               }
             }
             if constexpr (C::PASSES == 1) {
-              const n64_ptr pd = it.den + off * unsigned(ex ? a.nrhs * C::W0 : C::W0);
+              const n64_ptr pd = it.den + n64_off(off, ex && !C::TR ? a.nrhs * C::W0 : C::W0);
               const int64_t rstep = ex ? int64_t(C::W0) : kind == ITEM_UE ? rs_ue : rs_de;
 #pragma unroll
               for (int r = 0; r < NR; r++)
@@ -188,14 +192,14 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
                   rec[PO + r * C::W0 + s] =
                       r < a.nr ? pd[r * rstep + s] * (ex || C::TR ? weight64<KT>(pu, s) : weight64<KM>(pm, s)) : 0.0;
             } else if (pass == 0) {
-              const n64_ptr pd = it.den + off * unsigned(a.nrhs * C::W0);
+              const n64_ptr pd = it.den + n64_off(off, a.nrhs * C::W0);
 #pragma unroll
               for (int r = 0; r < NR; r++)
 #pragma unroll
                 for (int s = 0; s < C::W0; s++)
                   rec[PO + r * C::W0 + s] = r < a.nr ? pd[r * C::W0 + s] * weight64<KT>(pu, s) : 0.0;
             } else {
-              const n64_ptr pd = it.den + off * unsigned(C::W1);
+              const n64_ptr pd = it.den + n64_off(off, C::W1);
               const int64_t rstep = kind == ITEM_UE ? rs_ue : rs_de;
 #pragma unroll
               for (int r = 0; r < NR; r++)
