@@ -114,6 +114,7 @@ struct NearArgs {
   // caller's order (no separate scatter)
   const int* tperm;
   const double* tnor = nullptr;  // transposed near field: normals of the chunks' points
+  double padx = 1e18;            // FP64: x of the padding sources, at y = z = 0: no point lies there
   // Several right-hand sides: sden holds nrhs densities per source
   // (sden[(k * nrhs + r) * SD + s]); right-hand side r's equivalent densities
   // are rows r * nstride + node of UE and DE, and its values start at

@@ -1463,6 +1463,7 @@ int FMM3d::evaluate_impl(const double* d_src_den, double* d_trg_val, hipStream_t
   na.UE = ue_src; na.sz_ue = op.dat(UE);
   na.DE = de_d_.as<double>(); na.sz_de = op.dat(DE);
   na.tpos = tpos_d_.as<double>(); na.tval = tval_d_.as<double>();
+  na.padx = t.ctr[0] + (4 * t.rad0 + 1e18);
   na.nrhs = R;
   na.nstride = N;
   na.tstride = nt_ * TD;

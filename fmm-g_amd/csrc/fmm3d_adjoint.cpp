@@ -353,6 +353,7 @@ int FMM3d::evaluateAdjoint(const double* d_trg_in, double* d_src_out, hipStream_
   a.sam_ue = sam_d_[DC].as<double>(); a.n_ue = op.n_sam[DC]; a.UE = dc_d_.as<double>(); a.sz_ue = op.dat(DC);
   a.sam_de = sam_d_[UC].as<double>(); a.n_de = op.n_sam[UC]; a.DE = uc_d_.as<double>(); a.sz_de = op.dat(UC);
   a.tpos = spos_d_.as<double>(); a.tnor = snor_d_.as<double>();
+  a.padx = tree_.ctr[0] + (4 * tree_.rad0 + 1e18);
   a.tval = sden_d_.as<double>();
   a.nstride = N;
   // mixed, Laplace (a symmetric kernel): the forward FP32 near kernel

@@ -11,14 +11,14 @@
 // that one LDS read of a source serves two pairs.  Lanes form S copies of the
 // point pairs; copy c sweeps the block's sources c, c + S, ..., two at a time, the
 // same number of rounds for all copies (they run on into padding: zero density,
-// 1e18 away).  Neighbouring copies read neighbouring records, whose length is 32
-// bytes or an odd multiple of 16, so their reads fall into different banks (with
-// a contiguous share a copy, 8 copies met in one bank).  Pairs closer than the reference's 1e-8 cut
-// contribute nothing; the test is made only in blocks that hold the leaf's own
-// sources unless the host could not keep the other items 1e-7 away (see
-// NearChunk).  2.3e9 Laplace pairs (1M clustered points): 1.54 ms,
-// 4.36 with one point a lane, an item a staging round, square root and division;
-// 2.06 in leaf order instead of largest chunk first (the last chunks ran alone).
+// outside the domain).  Neighbouring copies read neighbouring records, whose length
+// is 32 bytes or an odd multiple of 16, so their reads fall into different banks
+// (with a contiguous share a copy, 8 copies met in one bank).  Pairs closer than the
+// reference's 1e-8 cut contribute nothing; the test is made only in blocks that hold
+// the leaf's own sources unless the host could not keep the other items 1e-7 away
+// (see NearChunk).  2.3e9 Laplace pairs (1M clustered points): 1.54 ms, 4.36 with one
+// point a lane, an item a staging round, square root and division; 2.06 in leaf order
+// instead of largest chunk first (the last chunks ran alone).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
   }
   // padding past the block
   if (lane < C::PAD - NB)
-    for (int e = 0; e < REC; e++) sh.rec[(NB + lane) * REC + e] = e == 0 ? 1e18 : 0.0;
+    for (int e = 0; e < REC; e++) sh.rec[(NB + lane) * REC + e] = e == 0 ? a.padx : 0.0;
   double acc[2][NR][OUT];
 #pragma unroll
   for (int q = 0; q < 2; q++)
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
                   rec[PO + r * C::W1 + s] = r < a.nr ? pd[r * rstep + s] * weight64<KM>(pm, s) : 0.0;
             }
           } else {
-            for (int e2 = 0; e2 < REC; e2++) rec[e2] = e2 == 0 ? 1e18 : 0.0;
+            for (int e2 = 0; e2 < REC; e2++) rec[e2] = e2 == 0 ? a.padx : 0.0;
           }
         }
         __syncthreads();

@@ -66,3 +66,22 @@ def test_direct_far_targets(gpu, kt):
     assert rel(out, ref) <= PARITY
     far = np.abs(np.repeat(chk, f.trg_dof, axis=0)).max(1) > 1e150
     assert np.abs(out[far] - ref[far]).max() <= 1e-140
+
+
+def test_domain_far_from_the_origin():
+    """A domain around (1e18, 0, 0) with a point there, a round place that the padding of
+    the packed sources must not have."""
+    n = 3000
+    c = np.array([1e18, 0.0, 0.0])
+    pos = c + 128.0 * np.random.default_rng(777).integers(-2 ** 33, 2 ** 33, (n, 3))
+    pos[7] = c
+    den = np.random.default_rng(778).standard_normal(n)
+    f = kifmm.FMM3d(111, [1.0, 0.25], 3, 40, 4, ctr=c, root_level=-40)
+    f.set_points(pos)
+    f.setup()
+    val = f.evaluate(den)
+    assert np.isfinite(val).all()
+    ops = O.Ops(111, [1.0, 0.25], 3, f.operator(0).reshape(98, 26).T, f.operator(1).reshape(26, 26).T)
+    tree = O.Tree(pos, None, ctr=c, root_level=-40, pts_max=40, max_level=4)
+    ref = O.evaluate(tree, ops, 111, [1.0, 0.25], pos, np.zeros_like(pos), pos, den, root_level=-40, ctr=c)
+    assert rel(val, ref) <= PARITY
