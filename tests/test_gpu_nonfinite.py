@@ -1,0 +1,50 @@
+"""GPU: densities that are not finite, or so large that their spectra may not be, in the
+FP64 pass.  The V-list sums take a group's sources without a look at their membership
+only if every one's transform input is finite (and below 1e290); otherwise member by
+member, so that a source adds nothing to the targets it is adjacent to.
+
+Against the CPU oracle: infinite, NaN and finite values at the same places, the finite
+ones within the FP64 parity bar (relative 2-norm 1e-12).
+"""
+import numpy as np
+import pytest
+
+import kifmm
+import oracle as O
+from kifmm import workloads as W
+from test_gpu_parity import PARITY, run_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def agree(val, ref):
+    for what in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(what(val), what(ref)), what.__name__
+    fin = np.isfinite(ref)
+    print("finite %d of %d, +inf %d, -inf %d" % (fin.sum(), ref.size, np.isposinf(ref).sum(), np.isneginf(ref).sum()),
+          flush=True)
+    if fin.any():
+        big = np.abs(ref[fin]).max()
+        d, s = (val[fin] / big) - (ref[fin] / big), ref[fin] / big
+        assert np.linalg.norm(d) <= PARITY * np.linalg.norm(s)
+
+
+# np 4: 1/G a power of two; 5: not, and frequency counts that no chunk divides.  Depth 2
+# and more: V lists on several levels; the group of the source, and groups beside it.
+@pytest.mark.parametrize("kt,np_,n,pts", [(111, 4, 1500, 8), (111, 5, 300, 8), (311, 4, 500, 12), (511, 5, 300, 12)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 1e294])
+def test_one_bad_density(kt, np_, n, pts, bad):
+    coefs = [1.0, 0.3]
+    pos = W.uniform(n, 780 + n)
+    sd = O.src_dof(kt)
+    rng = np.random.default_rng(781)
+    den = rng.standard_normal((3, n * sd))
+    den[1, (n // 3) * sd] = bad
+    f, val, ref = run_pair(kt, coefs, np_, pts, pos, np.zeros_like(pos), den[1])
+    agree(val, ref)
+    # three right-hand sides, one of them bad: the others are untouched
+    multi = f.evaluate_multi(den)
+    assert np.array_equal(multi[1], val, equal_nan=True)
+    for r in (0, 2):
+        assert np.isfinite(multi[r]).all()
+        assert np.array_equal(multi[r], f.evaluate(den[r]))
