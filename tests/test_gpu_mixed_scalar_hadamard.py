@@ -43,3 +43,33 @@ def test_tile_forms(gen, np_, n, pts, nrhs):
         assert np.array_equal(f.evaluate_multi(den)[nrhs - 1], val["mixed"])
     assert dual_gap(f, 755) < 1e-5
     assert rel(val["mixed"], val["fp64"]) < 1e-5
+
+
+# The two kernels of the mixed scalar V list give the same bits.  A launch of up to four
+# rounds of 512 workgroups (tiles of up to 32 groups x H / 8 frequencies x right-hand
+# sides) takes the matrix cores, a larger one whose tiles are not filled (24 groups a
+# tile) the vector unit's sweep.  Few groups on every level: at most a tile for five of
+# them (a tile holds 144 colleagues, a group has 26), so that one right-hand side surely
+# takes the former; at least a tile a level, so that many surely take the latter.
+@pytest.mark.parametrize("np_,nrhs,n,pts", [(4, 64, 300, 20), (6, 24, 300, 20), (8, 9, 900, 40), (6, 12, 700, 20)])
+def test_both_kernels_same_bits(np_, nrhs, n, pts):
+    H = (4 * np_ ** 3 + 4 + 15) // 16 * 16
+    if n == 700:  # a clustered tree: a few groups on each of several levels
+        pos = 0.37 + 0.6 * np.random.default_rng(756).random((n, 3)) ** 6
+    else:
+        pos = W.uniform(n, 757)
+    f = kifmm.FMM3d(111, [1.0, 0.25], np_, pts, 30, precision="mixed")
+    f.set_points(pos)
+    f.setup()
+    t = f.tree()
+    off = t["lists"]["v"][0]
+    groups = {(int(t["depth"][b]), int(t["parent"][b])) for b in range(len(off) - 1) if off[b + 1] > off[b]}
+    levels = np.bincount([d for d, _ in groups])
+    levels = levels[levels > 0]
+    print("groups a level", levels, flush=True)
+    assert ((levels + 4) // 5).sum() * (H // 8) <= 4 * 512
+    assert levels.sum() < 24 * len(levels) and len(levels) * (H // 8) * nrhs > 4 * 512
+    den = np.random.default_rng(758).standard_normal((nrhs, n))
+    multi = f.evaluate_multi(den)
+    for r in (0, nrhs // 2, nrhs - 1):
+        assert np.array_equal(multi[r], f.evaluate(den[r]))
