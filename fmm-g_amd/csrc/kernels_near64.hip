@@ -229,13 +229,15 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
                 double x = px[q] - s[0], y = py[q] - s[1], z = pz[q] - s[2];
                 const double r2 = fma(x, x, fma(y, y, z * z));
                 double inv = rsqrt64(r2);
-                if constexpr (CUT) inv = r2 < kMinDif * kMinDif ? 0.0 : inv;
+                const bool near = CUT && r2 < kMinDif * kMinDif;
+                if constexpr (!C::GRAD) inv = near ? 0.0 : inv;
                 if constexpr (C::TR) { x = -x; y = -y; z = -z; }  // the points are the sources
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
                   const double* w = s + PO + r * WK;
                   if constexpr (C::GRAD) {
-                    const double c = -w[0] * inv * (inv * inv);
+                    // (a cut pair's density is not looked at, finite or not)
+                    const double g = -w[0] * inv * (inv * inv), c = near ? 0.0 : g;
                     acc[q][r][0] = fma(c, x, acc[q][r][0]);
                     acc[q][r][1] = fma(c, y, acc[q][r][1]);
                     acc[q][r][2] = fma(c, z, acc[q][r][2]);

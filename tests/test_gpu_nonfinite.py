@@ -12,6 +12,7 @@ import pytest
 import kifmm
 import oracle as O
 from kifmm import workloads as W
+from test_gpu_adjoint import direct_grad
 from test_gpu_parity import PARITY, run_pair
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,22 @@ def test_one_bad_density(kt, np_, n, pts, bad):
     for r in (0, 2):
         assert np.isfinite(multi[r]).all()
         assert np.array_equal(multi[r], f.evaluate(den[r]))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_field_at_the_bad_source(bad, precision):
+    """A pair under the 1e-8 cut adds nothing to the gradient, whatever its density: the
+    bad source's own point keeps its finite gradient, every other point loses it."""
+    n, j = 150, 41
+    pos = W.uniform(n, 782)
+    den = np.random.default_rng(783).standard_normal(n)
+    den[j] = bad
+    f = kifmm.FMM3d(111, [1.0, 0.25], 4, n, 30, precision=precision)
+    f.set_points(0.5 * pos)
+    f.setup()
+    g = f.field(den).reshape(n, 3)
+    others = np.arange(n) != j
+    ref = direct_grad(0.5 * pos[others], den[others], 0.5 * pos[j:j + 1])[0]
+    assert np.linalg.norm(g[j] - ref) <= PARITY * np.linalg.norm(ref)
+    assert not np.isfinite(g[others]).any()
