@@ -859,6 +859,7 @@ __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t 
   constexpr bool NOR = needs_normals_ct(KT);
   constexpr int WO = NOR ? 6 : 3, REC = (WO + SD + 1) / 2 * 2;
   __shared__ __align__(16) double rec[256 * REC];
+  __shared__ int infs[4];
   const int tid = threadIdx.x;
   double tx[Q], ty[Q], tz[Q], acc[Q][TD];
 #pragma unroll
@@ -873,6 +874,7 @@ __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t 
   const int64_t j0 = int64_t(blockIdx.y) * chunk, j1 = j0 + chunk < ns ? j0 + chunk : ns;
   for (int64_t b = j0; b < j1; b += 256) {
     const int64_t j = b + tid;
+    bool inf = false;  // a density staged here is not finite (where that matters)
     __syncthreads();
     double* o = rec + tid * REC;
     if (j < j1) {
@@ -882,13 +884,32 @@ __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t 
         for (int d = 0; d < 3; d++) o[3 + d] = snor[3 * j + d];
       const int64_t k = sperm[j];
 #pragma unroll
-      for (int d = 0; d < SD; d++) o[WO + d] = sden[k * SD + d] * weight64<KT>(p, d);
+      for (int d = 0; d < SD; d++) {
+        o[WO + d] = sden[k * SD + d] * weight64<KT>(p, d);
+        if constexpr (both_signs64(KT, false)) inf = inf || !(fabs(sden[k * SD + d]) < INFINITY);
+      }
     } else {  // padding: far away, zero density
 #pragma unroll
       for (int d = 0; d < REC; d++) o[d] = d ? 0.0 : 1e18;
     }
+    if constexpr (both_signs64(KT, false)) infs[tid >> 6] = __any(inf);
     __syncthreads();
     const int cnt = j1 - b < 256 ? int(j1 - b) : 256;
+    if constexpr (both_signs64(KT, false)) {
+      inf = infs[0] | infs[1] | infs[2] | infs[3];
+#pragma unroll 1
+      for (int k = 0; inf && k < cnt; k++) {
+        const double* sr = rec + k * REC;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+          const double x = tx[q] - sr[0], y = ty[q] - sr[1], z = tz[q] - sr[2];
+          const double r2 = fma(x, x, fma(y, y, z * z));
+          const double inv = r2 < kMinDif * kMinDif ? 0.0 : rsqrt64(r2);
+          pair64_block<KT, false>(h, x, y, z, inv, sr + 3, sr + WO, acc[q]);
+        }
+      }
+      if (inf) continue;
+    }
     for (int k = 0; k < cnt; k++) {
       const double* sr = rec + k * REC;
 #pragma unroll

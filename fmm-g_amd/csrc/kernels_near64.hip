@@ -60,6 +60,7 @@ struct Near64 {
     int pre[kN64Win + 1];
     unsigned char kind[kN64Win];
     int wsum[2];
+    unsigned inf[2];
     union {
       Item item[kN64Win];
       double red[kN64Threads * 2 * OUT];
@@ -162,6 +163,7 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
         while (inext + 1 < nw && __builtin_amdgcn_readfirstlane(sh.pre[inext + 1]) <= base + NB) inext++;
         icur = inext;
         __syncthreads();
+        unsigned inf = 0;  // right-hand sides with a density here that is not finite (where that matters)
 #pragma unroll
         for (int e = 0; e < NS; e++) {
           const int slot = kN64Threads * e + lane;
@@ -188,16 +190,22 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
 #pragma unroll
               for (int r = 0; r < NR; r++)
 #pragma unroll
-                for (int s = 0; s < C::W0; s++)
-                  rec[PO + r * C::W0 + s] =
+                for (int s = 0; s < C::W0; s++) {
+                  const double v =
                       r < a.nr ? pd[r * rstep + s] * (ex || C::TR ? weight64<KT>(pu, s) : weight64<KM>(pm, s)) : 0.0;
+                  rec[PO + r * C::W0 + s] = v;
+                  if constexpr (both_signs64(KT, C::TR)) inf |= fabs(v) < INFINITY ? 0u : 1u << r;
+                }
             } else if (pass == 0) {
               const n64_ptr pd = it.den + n64_off(off, a.nrhs * C::W0);
 #pragma unroll
               for (int r = 0; r < NR; r++)
 #pragma unroll
-                for (int s = 0; s < C::W0; s++)
-                  rec[PO + r * C::W0 + s] = r < a.nr ? pd[r * C::W0 + s] * weight64<KT>(pu, s) : 0.0;
+                for (int s = 0; s < C::W0; s++) {
+                  const double v = r < a.nr ? pd[r * C::W0 + s] * weight64<KT>(pu, s) : 0.0;
+                  rec[PO + r * C::W0 + s] = v;
+                  if constexpr (both_signs64(KT, C::TR)) inf |= fabs(v) < INFINITY ? 0u : 1u << r;
+                }
             } else {
               const n64_ptr pd = it.den + n64_off(off, C::W1);
               const int64_t rstep = kind == ITEM_UE ? rs_ue : rs_de;
@@ -210,6 +218,12 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
           } else {
             for (int e2 = 0; e2 < REC; e2++) rec[e2] = e2 == 0 ? a.padx : 0.0;
           }
+        }
+        if constexpr (both_signs64(KT, C::TR)) {
+          unsigned any = 0;
+#pragma unroll
+          for (int r = 0; r < NR; r++) any |= __any(inf & (1u << r)) ? 1u << r : 0u;
+          sh.inf[lane >> 6] = any;
         }
         __syncthreads();
         if (!active) continue;
@@ -255,6 +269,30 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
         using FT = std::false_type;
         if (pass == 0) {
           const double h = ratio64<KT>(pu);
+          if constexpr (both_signs64(KT, C::TR)) {
+            const unsigned any = __builtin_amdgcn_readfirstlane(sh.inf[0] | sh.inf[1]);
+            if (any) {  // (the other right-hand sides keep their sums' bits)
+#pragma unroll 1
+              for (int i = 0; i < L; i++, rec += step)
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                  const double sg = C::TR ? -1.0 : 1.0;
+                  const double x = sg * (px[q] - rec[0]), y = sg * (py[q] - rec[1]), z = sg * (pz[q] - rec[2]);
+                  const double r2 = fma(x, x, fma(y, y, z * z));
+                  const double inv = r2 < kMinDif * kMinDif ? 0.0 : rsqrt64(r2);
+#pragma unroll
+                  for (int r = 0; r < NR; r++) {
+                    const double* n = C::TR ? pn[q] : rec + 3;
+                    const double* w = rec + PO + r * C::W0;
+                    if (any & (1u << r)) pair64_block<KT, C::TR>(h, x, y, z, inv, n, w, acc[q][r]);
+                    else if constexpr (C::TR) pair64_t<KT>(h, x, y, z, inv, n, w, acc[q][r]);
+                    else pair64<KT>(h, x, y, z, inv, n, w, acc[q][r]);
+                    __builtin_amdgcn_sched_barrier(0);
+                  }
+                }
+              continue;
+            }
+          }
           if (cut) sweep(std::integral_constant<int, KT>{}, TT{}, h);
           else sweep(std::integral_constant<int, KT>{}, FT{}, h);
         } else if constexpr (C::PASSES == 2) {

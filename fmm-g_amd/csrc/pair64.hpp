@@ -84,6 +84,30 @@ __device__ __forceinline__ void pair64(double h, double x, double y, double z, d
   }
 }
 
+// Whether the sums above (TR: those of the transpose below) form terms of both signs
+// from one density component: an infinite one would give NaN where the kernel block
+// times it is an infinity.
+__host__ __device__ constexpr bool both_signs64(int kt, bool tr) { return kt == 521 || (kt == 322 && !tr); }
+// The same pair with the block formed first, for densities that are not finite.
+template <int K, bool TR>
+__device__ __forceinline__ void pair64_block(double h, double x, double y, double z, double inv, const double* n,
+                                             const double* w, double* acc) {
+  const double v[3] = {x, y, z}, rn = dot3(x, y, z, n), inv2 = inv * inv, inv3 = inv2 * inv;
+  if constexpr (K == 322) {
+#pragma unroll
+    for (int s = 0; s < 3; s++) acc[0] += inv3 * fma(-3.0 * rn * inv2, v[s], n[s]) * w[s];
+  } else {
+    const double hi = h * inv3, g = inv3 * inv2 * rn;
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+      for (int s = 0; s < 3; s++) {
+        const double b = g * v[t] * v[s] + hi * (n[t] * v[s] - v[t] * n[s] + (t == s ? rn : 0.0));
+        acc[TR ? s : t] += b * w[TR ? t : s];
+      }
+  }
+}
+
 // acc += K(x; n)^T w, w per target DOF, acc per source DOF.
 template <int K>
 __device__ __forceinline__ void pair64_t(double h, double x, double y, double z, double inv, const double* n,
@@ -98,10 +122,10 @@ __device__ __forceinline__ void pair64_t(double h, double x, double y, double z,
       acc[1] = fma(g, y, acc[1]);
       acc[2] = fma(g, z, acc[2]);
     } else if constexpr (K == 322) {
-      const double a = inv3 * w[0], g = -3.0 * a * inv2 * dot3(x, y, z, n);
-      acc[0] = fma(a, n[0], fma(g, x, acc[0]));
-      acc[1] = fma(a, n[1], fma(g, y, acc[1]));
-      acc[2] = fma(a, n[2], fma(g, z, acc[2]));
+      const double a = inv3 * w[0], t = -3.0 * dot3(x, y, z, n) * inv2;
+      acc[0] = fma(fma(t, x, n[0]), a, acc[0]);
+      acc[1] = fma(fma(t, y, n[1]), a, acc[1]);
+      acc[2] = fma(fma(t, z, n[2]), a, acc[2]);
     } else if constexpr (K == 521) {
       const double rn = dot3(x, y, z, n), f = dot3(x, y, z, w), nw = dot3(n[0], n[1], n[2], w);
       const double hi = h * inv3, a = hi * rn, b = -hi * f, g = fma(inv3 * inv2 * rn, f, hi * nw);

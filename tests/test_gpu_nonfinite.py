@@ -68,3 +68,36 @@ def test_field_at_the_bad_source(bad, precision):
     ref = direct_grad(0.5 * pos[others], den[others], 0.5 * pos[j:j + 1])[0]
     assert np.linalg.norm(g[j] - ref) <= PARITY * np.linalg.norm(ref)
     assert not np.isfinite(g[others]).any()
+
+
+@pytest.mark.parametrize("kt", [121, 311, 312, 321, 322, 511, 521])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 1e294])
+def test_pair_sums(kt, bad):
+    """One box 1e-3 wide: near field, direct sum and transposed near field give an infinity
+    where the kernel block times the density does, and lose no finite value on the way."""
+    import torch
+    n, j, coefs = 150, 67, [1.0, 0.3]
+    pos = 0.3 + 1e-3 * W.uniform(n, 784)
+    rng = np.random.default_rng(785)
+    nor = rng.standard_normal((n, 3))
+    nor /= np.linalg.norm(nor, axis=1)[:, None]
+    f = kifmm.FMM3d(kt, coefs, 4, n, 30)
+    f.set_points(pos, nor)
+    f.setup()
+    den = rng.standard_normal(n * f.src_dof)
+    den[j * f.src_dof] = bad
+    ref = O.direct(kt, coefs, pos, nor, den, pos)
+    val = f.evaluate(den)
+    agree(val, ref)
+    good = rng.standard_normal((2, den.size))
+    multi = f.evaluate_multi(np.stack([good[0], den, good[1]]))
+    assert np.array_equal(multi[1], val, equal_nan=True)
+    assert np.array_equal(multi[0], f.evaluate(good[0])) and np.array_equal(multi[2], f.evaluate(good[1]))
+    out = torch.empty(n * f.trg_dof, dtype=torch.float64, device="cuda:0")
+    f.direct_device(torch.from_numpy(den).cuda(), torch.from_numpy(pos).cuda(), out)
+    agree(out.cpu().numpy(), ref)
+    w = rng.standard_normal(n * f.trg_dof)
+    w[j * f.trg_dof] = bad
+    M = O.kernel_matrix(kt, coefs, pos, nor, pos)
+    with np.errstate(invalid="ignore"):
+        agree(f.evaluate_adjoint(w), (M * w[:, None]).sum(0))
