@@ -21,6 +21,12 @@ struct NearChunk {
   int own = -1, unchk = 0;
 };
 constexpr int kNearChunk = 128;
+// The FP64 near kernels' workgroup, and the copies of a chunk's k points (two a lane)
+// on its lanes.
+constexpr int kN64Threads = 128, kN64Copies = 32;
+__host__ __device__ constexpr int near64_copies(int k) {
+  return kN64Threads / ((k + 1) / 2) < kN64Copies ? kN64Threads / ((k + 1) / 2) : kN64Copies;
+}
 // Right-hand sides per launch of the point kernels: groups of 1, 2, 4 or 8
 // (compile-time accumulator arrays); more go in several launches.
 constexpr int kMaxNr = 8;

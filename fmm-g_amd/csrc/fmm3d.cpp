@@ -383,13 +383,12 @@ int FMM3d::build_tasks() {
   std::vector<int64_t>& ioff = near_ioff_;
   std::vector<int64_t> coff(size_t(NL) + 1, 0);
   auto x_fallback = [&](int B) { return t.trg_num[B] * TD < szDC; };  // :1249
-  // the FP64 near kernels put two points a lane on 128 / ceil(k / 2) copies, so a
-  // leaf of 70 points leaves a fifth of the lanes idle and is cut in two; staging
-  // a source again costs about 0.03 of a sweep
+  // the FP64 near kernels put two points a lane (near64_copies), so a leaf of 70
+  // points leaves a fifth of the lanes idle and is cut in two; staging a source
+  // again costs about 0.03 of a sweep
   int max_tn = 0;
   for (int B : near_leaves) max_tn = std::max(max_tn, t.trg_num[B]);
-  auto copies64 = [](int k) { return std::min(32, kNearChunk / ((k + 1) / 2)); };
-  const std::vector<int> pick = split_leaves(max_tn, copies64, [](int, int) { return 1; }, 0.03);
+  const std::vector<int> pick = split_leaves(max_tn, near64_copies, [](int, int) { return 1; }, 0.03);
 #pragma omp parallel for schedule(dynamic, 256)
   for (int l = 0; l < NL; l++) {
     const int B = near_leaves[l], tn = t.trg_num[B];
@@ -443,7 +442,7 @@ int FMM3d::build_tasks() {
     }
     int64_t ci = coff[size_t(l)];
     for (int c = 0; c < tn; c += pick[tn - c]) {
-      near_cost[size_t(ci)] = float((exact + surf) / copies64(pick[tn - c]));
+      near_cost[size_t(ci)] = float((exact + surf) / near64_copies(pick[tn - c]));
       near_chunks_h_[size_t(ci++)] = make_near_chunk(B, c, pick[tn - c], ibeg, ni, true);
     }
     near_exact += double(tn) * exact;

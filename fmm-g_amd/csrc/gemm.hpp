@@ -120,7 +120,7 @@ __global__ __launch_bounds__(GT_T) void k_gemm_seq(GemmArgs g) {
       }
     }
   }
-  if (k0 < K) {  // the last K % 32 terms
+  if (k0 < K) {  // the last K % GT_K terms
 #pragma unroll
     for (int u = 0; u < GT_B; u++) Bs[buf][ks + u][js] = rb[u] * sct[sp + ks + u];
     __syncthreads();

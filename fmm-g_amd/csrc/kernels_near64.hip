@@ -29,7 +29,8 @@
 namespace kifmm {
 
 enum Near64Mode { NEAR64_VAL = 0, NEAR64_GRAD = 1, NEAR64_T = 2 };
-constexpr int kN64Threads = 128, kN64Win = 128, kN64Copies = 32;
+constexpr int kN64Win = 128;
+static_assert(kNearChunk <= kN64Threads, "a lane for every two points and more");
 typedef const __attribute__((address_space(1))) double* n64_ptr;
 // Offset of an item's source `row` among rows of `len` values.  64 bits: one leaf's
 // densities over all right-hand sides may pass 2^32 values.
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
   const NearChunk ch = a.chunks[a.order ? a.order[blockIdx.x] : int(blockIdx.x)];
   const int lane = threadIdx.x;
   const int tn = max(ch.tnum, 1), tl = (tn + 1) / 2;
-  const int S = min(kN64Threads / tl, kN64Copies);
+  const int S = near64_copies(tn);
   const int ti = lane % tl, sub = lane / tl;
   const bool active = sub < S;
   // points ti and ti + tl (absent: the first one again, not stored)

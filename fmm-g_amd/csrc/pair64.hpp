@@ -137,12 +137,6 @@ __device__ __forceinline__ void pair64_t(double h, double x, double y, double z,
       acc[0] = fma(a, w[0], fma(b, n[0], fma(g, x, acc[0])));
       acc[1] = fma(a, w[1], fma(b, n[1], fma(g, y, acc[1])));
       acc[2] = fma(a, w[2], fma(b, n[2], fma(g, z, acc[2])));
-    } else if constexpr (K == 301) {  // 4 source DOFs
-      const double f = dot3(x, y, z, w), g = inv3 * f;
-      acc[0] = fma(inv, w[0], fma(g, x, acc[0]));
-      acc[1] = fma(inv, w[1], fma(g, y, acc[1]));
-      acc[2] = fma(inv, w[2], fma(g, z, acc[2]));
-      acc[3] = fma(h, g, acc[3]);
     }
   }
 }
