@@ -61,18 +61,13 @@ __device__ __forceinline__ void pair64(double h, double x, double y, double z, d
     } else if constexpr (K == 322) {
       const double nw = dot3(n[0], n[1], n[2], w), rn = dot3(x, y, z, n);
       acc[0] = fma(inv3, fma(-3.0 * rn * inv2, dot3(x, y, z, w), nw), acc[0]);
-    } else if constexpr (K == 301 || K == 311) {
+    } else if constexpr (K == 301 || K == 311 || K == 511) {
       double f = dot3(x, y, z, w);
       if constexpr (K == 301) f += w[3];
-      const double g = inv3 * f;
-      acc[0] = fma(inv, w[0], fma(g, x, acc[0]));
-      acc[1] = fma(inv, w[1], fma(g, y, acc[1]));
-      acc[2] = fma(inv, w[2], fma(g, z, acc[2]));
-    } else if constexpr (K == 511) {
-      const double u = inv2 * dot3(x, y, z, w);  // (h w does not depend on the target)
-      acc[0] = fma(inv, fma(u, x, h * w[0]), acc[0]);
-      acc[1] = fma(inv, fma(u, y, h * w[1]), acc[1]);
-      acc[2] = fma(inv, fma(u, z, h * w[2]), acc[2]);
+      const double g = inv3 * f, c = K == 511 ? h * inv : inv;
+      acc[0] = fma(c, w[0], fma(g, x, acc[0]));
+      acc[1] = fma(c, w[1], fma(g, y, acc[1]));
+      acc[2] = fma(c, w[2], fma(g, z, acc[2]));
     } else if constexpr (K == 321) {
       const double g = inv3 * inv2 * dot3(x, y, z, n) * dot3(x, y, z, w);
       acc[0] = fma(g, x, acc[0]);
