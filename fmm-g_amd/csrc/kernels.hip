@@ -921,28 +921,34 @@ __global__ __launch_bounds__(256) void k_direct_part(KParams<double> p, int64_t 
       }
     }
   }
+  unsigned far = 0;  // targets to be summed again
 #pragma unroll
   for (int q = 0; q < Q; q++) {
     const int i = (int(blockIdx.x) * Q + q) * 256 + tid;
     if (i >= nt) continue;
-    if (!(tx[q] * tx[q] + ty[q] * ty[q] + tz[q] * tz[q] + src_r2 < 1e300)) {
-#pragma unroll
-      for (int d = 0; d < TD; d++) acc[q][d] = 0.0;
-#pragma unroll 1
-      for (int64_t j = j0; j < j1; j++) {
-        double blk[SD * TD], n[3] = {0.0, 0.0, 0.0};
-        if constexpr (NOR)
-          for (int d = 0; d < 3; d++) n[d] = snor[3 * j + d];
-        kblock<KT, double>(p, tx[q] - spos[3 * j], ty[q] - spos[3 * j + 1], tz[q] - spos[3 * j + 2], n[0], n[1], n[2], blk);
-        const double* w = sden + int64_t(sperm[j]) * SD;
-#pragma unroll
-        for (int d = 0; d < TD; d++)
-#pragma unroll
-          for (int e = 0; e < SD; e++) acc[q][d] += blk[d * SD + e] * w[e];
-      }
-    }
+    far |= tx[q] * tx[q] + ty[q] * ty[q] + tz[q] * tz[q] + src_r2 < 1e300 ? 0u : 1u << q;
 #pragma unroll
     for (int d = 0; d < TD; d++) part[(int64_t(blockIdx.y) * nt + i) * TD + d] = acc[q][d];
+  }
+#pragma unroll 1
+  for (int q = 0; far; q++, far >>= 1) {
+    const int i = (int(blockIdx.x) * Q + q) * 256 + tid;
+    if (!(far & 1)) continue;
+    const double* t = tpos + 3 * int64_t(i);
+    double v[TD] = {};
+#pragma unroll 1
+    for (int64_t j = j0; j < j1; j++) {
+      double blk[SD * TD], n[3] = {0.0, 0.0, 0.0};
+      if constexpr (NOR)
+        for (int d = 0; d < 3; d++) n[d] = snor[3 * j + d];
+      kblock<KT, double>(p, t[0] - spos[3 * j], t[1] - spos[3 * j + 1], t[2] - spos[3 * j + 2], n[0], n[1], n[2], blk);
+      const double* w = sden + int64_t(sperm[j]) * SD;
+#pragma unroll
+      for (int d = 0; d < TD; d++)
+#pragma unroll
+        for (int e = 0; e < SD; e++) v[d] += blk[d * SD + e] * w[e];
+    }
+    for (int d = 0; d < TD; d++) part[(int64_t(blockIdx.y) * nt + i) * TD + d] = v[d];
   }
 }
 

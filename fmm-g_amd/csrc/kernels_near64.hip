@@ -61,11 +61,11 @@ struct Near64 {
     int pre[kN64Win + 1];
     unsigned char kind[kN64Win];
     int wsum[2];
-    unsigned inf[2];
     union {
       Item item[kN64Win];
       double red[kN64Threads * 2 * OUT];
     };
+    unsigned inf[2];
   };
 };
 
@@ -164,7 +164,6 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
         while (inext + 1 < nw && __builtin_amdgcn_readfirstlane(sh.pre[inext + 1]) <= base + NB) inext++;
         icur = inext;
         __syncthreads();
-        unsigned inf = 0;  // right-hand sides with a density here that is not finite (where that matters)
 #pragma unroll
         for (int e = 0; e < NS; e++) {
           const int slot = kN64Threads * e + lane;
@@ -191,22 +190,16 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
 #pragma unroll
               for (int r = 0; r < NR; r++)
 #pragma unroll
-                for (int s = 0; s < C::W0; s++) {
-                  const double v =
+                for (int s = 0; s < C::W0; s++)
+                  rec[PO + r * C::W0 + s] =
                       r < a.nr ? pd[r * rstep + s] * (ex || C::TR ? weight64<KT>(pu, s) : weight64<KM>(pm, s)) : 0.0;
-                  rec[PO + r * C::W0 + s] = v;
-                  if constexpr (both_signs64(KT, C::TR)) inf |= fabs(v) < INFINITY ? 0u : 1u << r;
-                }
             } else if (pass == 0) {
               const n64_ptr pd = it.den + n64_off(off, a.nrhs * C::W0);
 #pragma unroll
               for (int r = 0; r < NR; r++)
 #pragma unroll
-                for (int s = 0; s < C::W0; s++) {
-                  const double v = r < a.nr ? pd[r * C::W0 + s] * weight64<KT>(pu, s) : 0.0;
-                  rec[PO + r * C::W0 + s] = v;
-                  if constexpr (both_signs64(KT, C::TR)) inf |= fabs(v) < INFINITY ? 0u : 1u << r;
-                }
+                for (int s = 0; s < C::W0; s++)
+                  rec[PO + r * C::W0 + s] = r < a.nr ? pd[r * C::W0 + s] * weight64<KT>(pu, s) : 0.0;
             } else {
               const n64_ptr pd = it.den + n64_off(off, C::W1);
               const int64_t rstep = kind == ITEM_UE ? rs_ue : rs_de;
@@ -221,7 +214,14 @@ __global__ __launch_bounds__(kN64Threads) void k_near64(NearArgs a, KParams<doub
           }
         }
         if constexpr (both_signs64(KT, C::TR)) {
-          unsigned any = 0;
+          // right-hand sides with a density here that is not finite
+          unsigned inf = 0, any = 0;
+#pragma unroll
+          for (int e = 0; e < NS; e++) {
+            const double* w = sh.rec + (kN64Threads * e + lane) * REC + PO;
+#pragma unroll
+            for (int i = 0; i < NR * C::W0; i++) inf |= fabs(w[i]) < INFINITY ? 0u : 1u << (i / C::W0);
+          }
 #pragma unroll
           for (int r = 0; r < NR; r++) any |= __any(inf & (1u << r)) ? 1u << r : 0u;
           sh.inf[lane >> 6] = any;

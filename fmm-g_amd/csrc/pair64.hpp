@@ -112,11 +112,18 @@ __device__ __forceinline__ void pair64_block(double h, double x, double y, doubl
 template <int K>
 __device__ __forceinline__ void pair64_t(double h, double x, double y, double z, double inv, const double* n,
                                          const double* w, double* acc) {
-  if constexpr (K == 111 || K == 121 || K == 311 || K == 321 || K == 511) {
+  if constexpr (K == 111 || K == 121 || K == 311 || K == 321) {
     pair64<K>(h, x, y, z, inv, n, w, acc);  // symmetric blocks
   } else {
     const double inv2 = inv * inv, inv3 = inv2 * inv;
-    if constexpr (K == 312) {
+    if constexpr (K == 511) {
+      // symmetric too; with one right-hand side h w, formed once for two points, is
+      // less than h / r a pair
+      const double u = inv2 * dot3(x, y, z, w);
+      acc[0] = fma(inv, fma(u, x, h * w[0]), acc[0]);
+      acc[1] = fma(inv, fma(u, y, h * w[1]), acc[1]);
+      acc[2] = fma(inv, fma(u, z, h * w[2]), acc[2]);
+    } else if constexpr (K == 312) {
       const double g = inv3 * w[0];
       acc[0] = fma(g, x, acc[0]);
       acc[1] = fma(g, y, acc[1]);
