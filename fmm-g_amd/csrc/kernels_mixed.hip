@@ -1249,7 +1249,8 @@ hipError_t launch_hadamard_mixed(const VlistArgs& v, const float2* dspec, const 
   // groups and more of 32: uniform 300,000 points, np 6, 567 and 766 us; Gaussians
   // 319 and 424), but thin lists (spheres; the sweep skips their empty places) only
   // from twelve rounds on (100,000 points 231 and 268; in between 30,000 points of
-  // six spheres 119 and 103).
+  // six spheres 119 and 103).  The thin window was measured at np 6 only; both kernels
+  // give the same bits, so that an edge elsewhere costs time alone.
   if (v.sd == 1 && v.td == 1 && v.mirror && v.mt_tiles > 0 && v.nrhs <= 65535) {
     const int64_t wgs = int64_t(v.mt_tiles) * (v.H / kMtF) * v.nrhs;
     if (wgs <= 4 * 512 || (v.ngrp >= 24 * int64_t(v.mt_tiles) && (!v.mt_thin || wgs >= 12 * 512))) {

@@ -52,7 +52,9 @@ struct Near64 {
   static constexpr int LEN = (3 + (SNOR ? 3 : 0) + WM + 1) / 2 * 2;
   static constexpr int REC = LEN > 4 && LEN % 4 == 0 ? LEN + 2 : LEN;  // doubles a staged source
   // sources a block: full rounds of the threads, within about 16 KB for one
-  // right-hand side; the same for more, whose sums then run in the same order
+  // right-hand side; the same for more, whose sums then run in the same order (up to
+  // 77 KB with eight: two workgroups a CU.  2.8M points, 511: 48 ms, and 43 with the
+  // kernel before, which staged 128 sources and formed a pair's block once for all)
   static constexpr int NB = 3 + (SNOR ? 3 : 0) + WM / NR <= 6 ? 256 : 128;
   static constexpr int PAD = NB + 2 * kN64Copies;
   struct Item { double cw[4]; n64_ptr pos, den, nor; };

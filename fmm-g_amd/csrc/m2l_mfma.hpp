@@ -18,12 +18,13 @@
 // are one register a chain, a lane an entry, and the broadcast of one 4-row block
 // picks the source child.  Past the staging no wave waits for another.
 //
-// Bound by the matrix cores (busy half of the time) and, not hidden, by the staging
-// and the LDS gathers between the products.  Laplace np 6: 8 million points 5.43 ->
-// 4.05 ms, a million uniform points 757 -> 517 us, 100,000 points 164 -> 117 us.
-// With the offset's spectra gathered from the table by every wave, or staged by the
-// workgroup behind a barrier an offset: 4.3 ms; child spectra staged in batches of
-// eight loads: 4.9 ms.
+// Bound by the matrix cores (busy 60% of the time) and, not hidden, by the staging
+// and the LDS gathers between the products (half of the LDS cycles are bank
+// conflicts).  Laplace np 6: 8 million points 5.05 -> 3.53 ms in a run of passes (5.43
+// -> 4.05 in the kernel trace of a few), a million uniform points 757 -> 517 us,
+// 100,000 points 164 -> 117 us.  In that trace, with the offset's spectra gathered from
+// the table by every wave, or staged by the workgroup behind a barrier an offset: 4.3
+// ms; child spectra staged in batches of eight loads: 4.9 ms.
 #pragma once
 #include <hip/hip_runtime.h>
 
